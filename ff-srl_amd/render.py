@@ -141,9 +141,9 @@ class RaycastRendererDO:
         self.camera.mode = int(render_mode)
 
     def set_traversal(self, traversal: int) -> None:
-        """0 picks by image size (2x2-ray quads per lane from 128x128 pixels,
-        one ray per lane below), 1 one ray per lane, 2 quads.  The images are
-        the same bit for bit."""
+        """0: a wavefront walks the BVH for a block of rays (the default), 1
+        one ray per lane, 2 a lane per pixel's 2x2 rays.  The images are the
+        same bit for bit."""
         self.traversal = int(traversal)
         self.camera.traversal = self.traversal
 

@@ -174,14 +174,16 @@ typedef struct ffsrl_camera {
                                      colours where a triangle has none), 5 per-triangle colour */
   float light_dir[3];
   float light_intensity;
-  int32_t traversal;              /* FFSRL_TRAVERSE_*: 0 (zero-initialised) picks by image size */
+  int32_t traversal;              /* FFSRL_TRAVERSE_*: 0 (zero-initialised) is automatic */
 } ffsrl_camera;
 
-/* Ray traversal of the renderer.  Both forms give the same hits, depths and
- * colours bit for bit; they differ only in speed.  PER_RAY: a lane traces
- * one supersampled ray.  QUAD: a lane traces the 2x2 rays of its pixel with
- * one stack (a BVH of at most 2^28 - 1 nodes).  AUTO: QUAD from 128x128
- * output pixels, PER_RAY below. */
+/* Ray traversal of the renderer.  All forms give the same hits, depths and
+ * colours bit for bit; they differ only in speed.  AUTO: a wavefront walks the
+ * BVH once for a block of rays (8x8 to 16x16, by the size of the launch); it is
+ * fastest for a pinhole table of directions, and traces the rays of any other
+ * one by one.  PER_RAY: a lane traces one supersampled ray.  QUAD: a lane
+ * traces the 2x2 rays of its pixel with one stack (a BVH of at most 2^28 - 1
+ * nodes, which AUTO asks for too from 128x128 output pixels). */
 #define FFSRL_TRAVERSE_AUTO 0
 #define FFSRL_TRAVERSE_PER_RAY 1
 #define FFSRL_TRAVERSE_QUAD 2
