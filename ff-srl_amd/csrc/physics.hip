@@ -64,13 +64,25 @@ constexpr int kMaxFrameVertices = (kLdsBytes - 512) / 16;
 // (FFSRL_STATUS_SATURATED): the frame then no longer equals the plain form,
 // which sums floats.
 //
-// A vertex owns 16 B of LDS, two 64-bit words updated with ds_add_u64:
-//   w0 = X + Y * 2^32,  w1 = Z + count * 2^32   (two's complement, mod 2^64)
-// where X, Y, Z are the int32 fixed-point sums.  Integer addition mod 2^64 is
-// exact and associative, so w0 and w1 hold exactly these values whatever the
-// order; since |X| < 2^31, X is the low half of w0 read as int32 and
-// Y = high half - (X < 0 ? -1 : 0) (likewise Z and the count).  One 64-bit
-// atomic thus carries two sums at one address.
+// A vertex owns 16 B of LDS, two 64-bit words updated with ds_add_u64.  With
+// X, Y, Z the int32 fixed-point sums of its k terms they are, mod 2^64,
+//   w0 = (X + k B) + (Y + k B) 2^32,  w1 = (Z + k B) + H 2^32,
+//   H  = count + k 2^12 + marks 2^24,
+// where B is the bit pattern of 1.5 * 2^23: for |v| <= 2^22 the float
+// v + 1.5 * 2^23 is v rounded to the nearest integer (ties to even) and its
+// bits are B + that integer, so one float add rounds, converts and biases a
+// component, and a biased component is a positive word that needs no sign
+// borrow when two are paired.  A term costs 3 adds and a compare shared by its
+// constraint instead of round, convert, clamp, mark and two sign borrows per
+// vertex (a tet's four vertices 73 -> 31 vector instructions, an edge's two
+// 46 -> 25), and the sums are the same integers.  Larger terms take the
+// clamping conversion (lds_acc), with the same bias.  The reader takes k from
+// w1's high word (the biased low sums carry at most 0.3 k into it, and the
+// counts add at most 2 k, both below 2^12), subtracts k B, and decodes: X is
+// the low half of w0 read as int32 and Y = high half - (X < 0 ? -1 : 0)
+// (likewise Z and H).  Integer addition mod 2^64 is exact and associative, so
+// the words hold exactly these values whatever the order.  One 64-bit atomic
+// thus carries two sums at one address.
 constexpr float kFixMax = 16777215.0f;  // 2^24 - 1 quanta
 
 struct FrameCtx {
@@ -89,22 +101,19 @@ __device__ __forceinline__ NHConst uniform(NHConst k) {
   return NHConst{uniform(k.gamma), uniform(k.alpha_h), uniform(k.alpha_d)};
 }
 
-// A term that left the range or was not finite adds kSatMark to its count
-// (counts stay below 2^16: at most FFSRL_MAX_TERMS terms of weight <= 2), so
-// the apply phase sees it in the sum's count and sets the workgroup's
-// saturation flag (one LDS word, cleared and read once per env frame); no
-// register holds a flag across the projection loops.
-constexpr uint32_t kSatMark = 1u << 16;
+constexpr float kBias = 12582912.0f;        // 1.5 * 2^23
+constexpr uint32_t kBiasBits = 0x4B400000u;  // its bits (B above)
+constexpr float kBiasMax = 4194304.0f;      // 2^22: the sum stays in [2^23, 2^24], where one ulp is one quantum
+constexpr uint32_t kTermOne = 1u << 12;     // one term, in w1's high word
+// A term that left the range or was not finite adds kSatMark as well, so the
+// apply phase sees it in the sum and sets the workgroup's saturation flag (one
+// LDS word, cleared and read once per env frame); no register holds a flag
+// across the projection loops.
+constexpr uint32_t kSatMark = 1u << 24;
 
 __device__ __forceinline__ int& sat_flag() {
   __shared__ int flag;
   return flag;
-}
-
-// The count of a decoded sum without saturation marks; raises the flag.
-__device__ __forceinline__ int32_t sum_count(int32_t n) {
-  if (__builtin_expect((uint32_t)n >= kSatMark, 0)) sat_flag() = 1;
-  return n & (int32_t)(kSatMark - 1u);
 }
 
 __device__ __forceinline__ int32_t to_fix(float v) {
@@ -112,27 +121,56 @@ __device__ __forceinline__ int32_t to_fix(float v) {
   v = fminf(fmaxf(v, -kFixMax), kFixMax);
   return (int32_t)v;
 }
-// (lo + hi * 2^32) as a 64-bit two's complement addend, lo sign-extended.
-__device__ __forceinline__ unsigned long long pack2(int32_t lo, int32_t hi) {
-  const uint32_t h = (uint32_t)hi + (uint32_t)(lo >> 31);
-  return ((unsigned long long)h << 32) | (uint32_t)lo;
-}
+// w = lo + hi * 2^32 with lo a signed 32-bit value.
 __device__ __forceinline__ void unpack2(unsigned long long w, int32_t* lo, int32_t* hi) {
   const int32_t l = (int32_t)(uint32_t)w;
   *lo = l;
   *hi = (int32_t)((uint32_t)(w >> 32) - (uint32_t)(l >> 31));
 }
-// Adds sign * d (given in quanta: the delta times c.inv_q) to the fixed-point
-// sums of vertex i and n to its count.
-template <int SIGN>
-__device__ __forceinline__ void lds_acc(const FrameCtx& c, int i, f3 d, uint32_t n) {
-  const float sx = d.x, sy = d.y, sz = d.z;
-  // IEEE 754-2019 maximum propagates NaN, which fails the comparison
-  const float m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(sx), fabsf(sy)), fabsf(sz));
-  const uint32_t mark = m <= kFixMax ? 0u : kSatMark;
-  const int32_t x = to_fix(sx), y = to_fix(sy), z = to_fix(sz);
-  atomicAdd(&c.acc[2 * i], pack2(SIGN * x, SIGN * y));
-  atomicAdd(&c.acc[2 * i + 1], pack2(SIGN * z, (int32_t)(n + mark)));
+// The sums and the count of a vertex's words; raises the saturation flag.
+__device__ __forceinline__ void decode_sums(unsigned long long w0, unsigned long long w1, int32_t* fx, int32_t* fy,
+                                            int32_t* fz, int32_t* n) {
+  const uint32_t k = ((uint32_t)(w1 >> 32) / kTermOne) % (kSatMark / kTermOne);
+  const unsigned long long bias = (unsigned long long)k * kBiasBits;
+  int32_t h;
+  unpack2(w0 - bias - (bias << 32), fx, fy);
+  unpack2(w1 - bias, fz, &h);
+  if (__builtin_expect((uint32_t)h >= kSatMark, 0)) sat_flag() = 1;
+  *n = h & (int32_t)(kTermOne - 1u);
+}
+// Adds the K vertex terms d (given in quanta: the deltas times c.inv_q) of one
+// constraint to the fixed-point sums of vertices i and n to their counts.
+template <int K>
+__device__ __forceinline__ void lds_acc(const FrameCtx& c, const int (&i)[K], const f3 (&d)[K], uint32_t n) {
+  // IEEE 754-2019 maximum propagates NaN, which fails the comparisons
+  float m = 0.0f;
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    m = __builtin_elementwise_maximum(
+        __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, fabsf(d[k].x)), fabsf(d[k].y)), fabsf(d[k].z));
+  uint32_t h = n + kTermOne;
+  uint32_t x[K], y[K], z[K];
+  if (__builtin_expect(m <= kBiasMax, 1)) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      x[k] = __float_as_uint(d[k].x + kBias);
+      y[k] = __float_as_uint(d[k].y + kBias);
+      z[k] = __float_as_uint(d[k].z + kBias);
+    }
+  } else {
+    if (!(m <= kFixMax)) h += kSatMark;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      x[k] = kBiasBits + (uint32_t)to_fix(d[k].x);
+      y[k] = kBiasBits + (uint32_t)to_fix(d[k].y);
+      z[k] = kBiasBits + (uint32_t)to_fix(d[k].z);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    atomicAdd(&c.acc[2 * i[k]], ((unsigned long long)y[k] << 32) | x[k]);
+    atomicAdd(&c.acc[2 * i[k] + 1], ((unsigned long long)h << 32) | z[k]);
+  }
 }
 
 __device__ __forceinline__ float4 with_w(f3 a, float w) { return make_float4(a.x, a.y, a.z, w); }
@@ -234,10 +272,7 @@ __device__ __forceinline__ void process_tet(const ffsrl_batch& b, const ffsrl_pa
     }
   }
   if (n) {
-    lds_acc<1>(c, tc.q.x, d[0], n);
-    lds_acc<1>(c, tc.q.y, d[1], n);
-    lds_acc<1>(c, tc.q.z, d[2], n);
-    lds_acc<1>(c, tc.q.w, d[3], n);
+    lds_acc<4>(c, {tc.q.x, tc.q.y, tc.q.z, tc.q.w}, d, n);
   }
 }
 
@@ -258,8 +293,7 @@ __device__ __forceinline__ void process_edge(const ffsrl_batch& b, const ffsrl_p
     if (CARRY && (ok || fresh)) b.lam_e[e.lam_ebase + j] = lam;
   }
   if (ok) {
-    lds_acc<-1>(c, ec.q.x, d * A.w, 1u);
-    lds_acc<1>(c, ec.q.y, d * B.w, 1u);
+    lds_acc<2>(c, {ec.q.x, ec.q.y}, {-(d * A.w), d * B.w}, 1u);
   }
 }
 
@@ -456,9 +490,9 @@ __device__ __forceinline__ void collide_tris(const ffsrl_batch& b, const ffsrl_p
     }
     if (len > 0.0f) {
       atomicAdd(contacts, 1);
-      if (A.w > 0.0f) lds_acc<-1>(c, t.x, r[0] * c.inv_q, 0u);
-      if (B.w > 0.0f) lds_acc<-1>(c, t.y, r[1] * c.inv_q, 0u);
-      if (Cc.w > 0.0f) lds_acc<-1>(c, t.z, r[2] * c.inv_q, 0u);
+      if (A.w > 0.0f) lds_acc<1>(c, {t.x}, {-(r[0] * c.inv_q)}, 0u);
+      if (B.w > 0.0f) lds_acc<1>(c, {t.y}, {-(r[1] * c.inv_q)}, 0u);
+      if (Cc.w > 0.0f) lds_acc<1>(c, {t.z}, {-(r[2] * c.inv_q)}, 0u);
     }
   }
 }
@@ -554,9 +588,7 @@ __device__ __forceinline__ void frame_env(const ffsrl_batch& b, const ffsrl_para
         c.acc[2 * i] = 0ull;
         c.acc[2 * i + 1] = 0ull;
         int32_t fx, fy, fz, n;
-        unpack2(w0, &fx, &fy);
-        unpack2(w1, &fz, &n);
-        n = sum_count(n);
+        decode_sums(w0, w1, &fx, &fy, &fz, &n);
         float4 p4 = ld4(P, vb + i);
         f3 p = xyz(p4);
         if (n > 0) {
@@ -581,9 +613,7 @@ __device__ __forceinline__ void frame_env(const ffsrl_batch& b, const ffsrl_para
           c.acc[2 * i + 1] = 0ull;
           if (!last_it && (w0 | w1) == 0ull) continue;
           int32_t fx, fy, fz, n;
-          unpack2(w0, &fx, &fy);
-          unpack2(w1, &fz, &n);
-          (void)sum_count(n);  // collision terms carry no count, only saturation marks
+          decode_sums(w0, w1, &fx, &fy, &fz, &n);  // collision terms carry no count, only saturation marks
           const float4 p4 = ld4(P, vb + i);
           const f3 p = xyz(p4) + mk((float)fx, (float)fy, (float)fz) * c.q;
           if (last_it)
@@ -799,7 +829,7 @@ __device__ __forceinline__ bool share_wait(uint32_t* ctr, uint32_t target) {
 
 // The env's share of one workgroup: chunks until the env's counter runs out.
 template <int BLOCK, bool CARRY, bool COLLIDE>
-__device__ void share_env(const ffsrl_batch& b, const ffsrl_params& prm, const ShareWs& ws, int el, int env,
+__device__ __forceinline__ void share_env(const ffsrl_batch& b, const ffsrl_params& prm, const ShareWs& ws, int el, int env,
                           int refit, unsigned long long* lds) {
   __shared__ int s_chunk, s_ok, s_last, s_contacts;
   const ffsrl_env_desc e = b.envs[env];
@@ -910,9 +940,7 @@ __device__ void share_env(const ffsrl_batch& b, const ffsrl_params& prm, const S
         if (w0) gacc[2 * i] = 0ull;
         if (w1) gacc[2 * i + 1] = 0ull;
         int32_t fx, fy, fz, n;
-        unpack2(w0, &fx, &fy);
-        unpack2(w1, &fz, &n);
-        n = sum_count(n);
+        decode_sums(w0, w1, &fx, &fy, &fz, &n);
         const float4 p4 = ld4c(P, vb + i);
         f3 p = xyz(p4);
         if (n > 0) {
@@ -933,9 +961,7 @@ __device__ void share_env(const ffsrl_batch& b, const ffsrl_params& prm, const S
         if (w1) gacc[2 * i + 1] = 0ull;
         if (!last_it && (w0 | w1) == 0ull) continue;
         int32_t fx, fy, fz, n;
-        unpack2(w0, &fx, &fy);
-        unpack2(w1, &fz, &n);
-        (void)sum_count(n);  // collision terms carry no count, only saturation marks
+        decode_sums(w0, w1, &fx, &fy, &fz, &n);  // collision terms carry no count, only saturation marks
         const float4 p4 = ld4c(P, vb + i);
         const f3 p = xyz(p4) + mk((float)fx, (float)fy, (float)fz) * c.q;
         if (last_it)
@@ -988,9 +1014,7 @@ __device__ __forceinline__ float4 fold_advance(const FrameCtx& c, const VertexSt
                                                unsigned long long w0, unsigned long long w1, float dr, bool boundary,
                                                float4 x4, float4* xs) {
   int32_t fx, fy, fz, n;
-  unpack2(w0, &fx, &fy);
-  unpack2(w1, &fz, &n);
-  n = sum_count(n);
+  decode_sums(w0, w1, &fx, &fy, &fz, &n);
   f3 p = xyz(p4);
   if (n > 0) {
     const float s = c.q * __builtin_amdgcn_rcpf((float)n);
@@ -1005,7 +1029,7 @@ __device__ __forceinline__ float4 fold_advance(const FrameCtx& c, const VertexSt
 }
 
 template <int BLOCK, bool CARRY>
-__device__ void share_fold_env(const ffsrl_batch& b, const ffsrl_params& prm, const ShareWs& ws, int el, int env,
+__device__ __forceinline__ void share_fold_env(const ffsrl_batch& b, const ffsrl_params& prm, const ShareWs& ws, int el, int env,
                                int refit, unsigned long long* lds) {
   __shared__ int s_chunk, s_ok, s_last;
   const ffsrl_env_desc e = b.envs[env];
@@ -1179,9 +1203,7 @@ __device__ void share_fold_env(const ffsrl_batch& b, const ffsrl_params& prm, co
       unsigned long long* g2 = U >= 2 ? sums(last - 1) : nullptr;
       for (int i = v0 + tid; i < v1; i += BLOCK) {
         int32_t fx, fy, fz, n;
-        unpack2(ldu64c(g, 2 * i), &fx, &fy);
-        unpack2(ldu64c(g, 2 * i + 1), &fz, &n);
-        n = sum_count(n);
+        decode_sums(ldu64c(g, 2 * i), ldu64c(g, 2 * i + 1), &fx, &fy, &fz, &n);
         const float4 p4 = ld4c(P, i);
         f3 p = xyz(p4);
         if (n > 0) {
@@ -1417,7 +1439,7 @@ constexpr int kSoloMaxVertices = (kLdsBytes - kPartStaticLds) / kSoloBytes;
 // weights stay in the model's arrays as there.  Each pass has no exchange and
 // no wait; the model's p is written once, after the last pass.
 template <bool CARRY, bool COLLIDE>
-__device__ void solo_env(const ffsrl_batch& b, const ffsrl_params& prm, const PartsWs& ws, int env, int refit,
+__device__ __forceinline__ void solo_env(const ffsrl_batch& b, const ffsrl_params& prm, const PartsWs& ws, int env, int refit,
                          unsigned long long* lds) {
   constexpr int BLOCK = 1024;
   const ffsrl_env_desc e = b.envs[env];
@@ -1482,9 +1504,7 @@ __device__ void solo_env(const ffsrl_batch& b, const ffsrl_params& prm, const Pa
         lds[2 * i] = 0ull;
         lds[2 * i + 1] = 0ull;
         int32_t fx, fy, fz, n;
-        unpack2(w0, &fx, &fy);
-        unpack2(w1, &fz, &n);
-        n = sum_count(n);
+        decode_sums(w0, w1, &fx, &fy, &fz, &n);
         const float4 p4 = Pl[i];
         f3 p = xyz(p4);
         if (n > 0) {
@@ -1515,9 +1535,7 @@ __device__ void solo_env(const ffsrl_batch& b, const ffsrl_params& prm, const Pa
           lds[2 * i + 1] = 0ull;
           if (!last_it && (w0 | w1) == 0ull) continue;
           int32_t fx, fy, fz, n;
-          unpack2(w0, &fx, &fy);
-          unpack2(w1, &fz, &n);
-          (void)sum_count(n);  // collision terms carry no count, only saturation marks
+          decode_sums(w0, w1, &fx, &fy, &fz, &n);  // collision terms carry no count, only saturation marks
           const float4 p4 = Pl[i];
           const f3 p = xyz(p4) + mk((float)fx, (float)fy, (float)fz) * c.q;
           if (last_it)
@@ -1546,7 +1564,7 @@ __device__ void solo_env(const ffsrl_batch& b, const ffsrl_params& prm, const Pa
 // its copy of a shared vertex, and the owner clears plane (x - 1) % 3, which
 // every part has read before arriving at exchange x.
 template <bool CARRY, bool COLLIDE>
-__device__ void part_env(const ffsrl_batch& b, const ffsrl_params& prm, const PartsWs& ws, int env, int pi, int np,
+__device__ __forceinline__ void part_env(const ffsrl_batch& b, const ffsrl_params& prm, const PartsWs& ws, int env, int pi, int np,
                          int refit, unsigned long long* lds) {
   constexpr int BLOCK = 1024;
   constexpr int E = COLLIDE ? 2 : 1;  // exchanges per pass
@@ -1669,9 +1687,7 @@ __device__ void part_env(const ffsrl_batch& b, const ffsrl_params& prm, const Pa
       unsigned long long w0, w1;
       take(i, m, gs, old, &w0, &w1);
       int32_t fx, fy, fz, n;
-      unpack2(w0, &fx, &fy);
-      unpack2(w1, &fz, &n);
-      n = sum_count(n);
+      decode_sums(w0, w1, &fx, &fy, &fz, &n);
       const float4 p4 = Pl[i];
       f3 p = xyz(p4);
       if (n > 0) {
@@ -1702,9 +1718,7 @@ __device__ void part_env(const ffsrl_batch& b, const ffsrl_params& prm, const Pa
         take(i, m, gc, oc, &w0, &w1);
         if (!last_it && (w0 | w1) == 0ull) continue;
         int32_t fx, fy, fz, n;
-        unpack2(w0, &fx, &fy);
-        unpack2(w1, &fz, &n);
-        (void)sum_count(n);  // collision terms carry no count, only saturation marks
+        decode_sums(w0, w1, &fx, &fy, &fz, &n);  // collision terms carry no count, only saturation marks
         const float4 p4 = Pl[i];
         const f3 p = xyz(p4) + mk((float)fx, (float)fy, (float)fz) * c.q;
         if (last_it)
