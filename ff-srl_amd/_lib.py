@@ -132,6 +132,7 @@ SIGNATURES = {
     "ffsrl_instrument_cartesian": [_P(Batch), _P(Instrument), _vp, _vp, _vp, _vp],
     "ffsrl_instrument_set_rcm": [_P(Batch), _P(Instrument), _vp, _vp, _vp],
     "ffsrl_instrument_update": [_P(Batch), _P(Instrument), _vp],
+    "ffsrl_reset_envs": [_P(Batch), _P(Instrument), _vp, _vp, _vp, _vp, _vp, _i32, _vp],
     "ffsrl_bvh_build_device": [_vp, _i32, _i32, _vp],
     "ffsrl_bounds_integrate": [_P(Batch), _P(Params), _i32, _i32, _vp],
     "ffsrl_zero_lambdas": [_P(Batch), _i32, _i32, _vp],

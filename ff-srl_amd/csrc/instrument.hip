@@ -342,6 +342,45 @@ __global__ void k_instrument_grasp(ffsrl_batch b, float radius, const int32_t* s
   b.drag[g] = dr;
 }
 
+// Environments of one reset launch, passed by value: no copy of the list to
+// the device and no wait for one (2,000 B of the 4 KiB of kernel arguments).
+constexpr int kResetIds = 500;
+struct ResetIds {
+  int32_t env[kResetIds];
+};
+struct ResetFrom {
+  const float *x, *tips, *bases, *xform;
+};
+
+// Block (x, k): vertices x*256.. of the k-th listed env, its instrument state
+// by block x = 0.  Bound by the 52 B written and 16 B read per vertex; one
+// launch for the list, where one tensor operation per env and array is host
+// time (half of 256 liver scenes: 7,790 -> 43 us for the reset and refit).
+__global__ void k_reset_envs(ffsrl_batch b, ffsrl_instrument ins, ResetFrom from, ResetIds ids) {
+  const int env = ids.env[blockIdx.y];
+  const ffsrl_env_desc e = b.envs[env];
+  const int t = threadIdx.x, i = blockIdx.x * blockDim.x + t;
+  if (i < e.nv) {
+    const int64_t g = (int64_t)e.vbase + i;
+    const float4 x = ld4(from.x, g);
+    st4(b.x, g, x);
+    st4(b.p, g, make_float4(0.0f, 0.0f, 0.0f, x.w));
+    st4(b.v, g, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+    b.drag[g] = 0.0f;
+  }
+  if (blockIdx.x) return;
+  if (t < 12) {
+    b.tips[env * 12 + t] = from.tips[env * 12 + t];
+    b.caps_base[env * 12 + t] = from.bases[env * 12 + t];
+  }
+  if (!from.xform) return;
+  if (t < 112) ins.xform[env * 112 + t] = from.xform[env * 112 + t];
+  if (t < 3) {
+    ins.drag_cut_heat[env * 3 + t] = 0;
+    ins.drag_cut_heat_update[env * 3 + t] = 0;
+  }
+}
+
 int check(const ffsrl_batch* b, const ffsrl_instrument* ins) {
   if (!b || !ins) return fail(FFSRL_E_ARG, "instrument: NULL batch or instrument");
   if (!ins->xform || !ins->height || !b->tips) return fail(FFSRL_E_ARG, "instrument: NULL transforms, heights or tips");
@@ -408,6 +447,34 @@ int ffsrl_instrument_update(const ffsrl_batch* b, const ffsrl_instrument* ins, v
   if (rc) return rc;
   if (ins->n_env == 0) return 0;
   hipLaunchKernelGGL(k_instrument_update, env_grid(ins->n_env), dim3(64), 0, as_stream(stream), *b, *ins);
+  FFSRL_HIP(hipGetLastError());
+  return 0;
+}
+
+int ffsrl_reset_envs(const ffsrl_batch* b, const ffsrl_instrument* ins, const float* x0, const float* tips0,
+                     const float* bases0, const float* xform0, const int32_t* envs, int32_t n, void* stream) {
+  if (!b) return fail(FFSRL_E_ARG, "reset: batch NULL");
+  if (!b->envs || !b->x || !b->p || !b->v || !b->drag || !b->tips || !b->caps_base || !x0 || !tips0 || !bases0)
+    return fail(FFSRL_E_ARG, "reset: NULL state, instrument points or initial state");
+  if (ins) {
+    const int rc = check(b, ins);
+    if (rc) return rc;
+    if (!xform0 || !ins->drag_cut_heat || !ins->drag_cut_heat_update)
+      return fail(FFSRL_E_ARG, "reset: NULL initial transforms or clamp state");
+  }
+  if (n < 0 || (n > 0 && !envs)) return fail(FFSRL_E_ARG, "reset: %d environments listed, list %p", n, (const void*)envs);
+  for (int32_t i = 0; i < n; ++i)
+    if (envs[i] < 0 || envs[i] >= b->n_env)
+      return fail(FFSRL_E_ARG, "reset: environment %d of %d", envs[i], b->n_env);
+  const ffsrl_instrument none = {};
+  const ResetFrom from{x0, tips0, bases0, ins ? xform0 : nullptr};
+  const unsigned gx = (unsigned)((b->max_nv < 1 ? 1 : b->max_nv) + 255) / 256;
+  for (int32_t k = 0; k < n; k += kResetIds) {
+    const int32_t m = n - k < kResetIds ? n - k : kResetIds;
+    ResetIds ids;
+    for (int32_t i = 0; i < m; ++i) ids.env[i] = envs[k + i];
+    hipLaunchKernelGGL(k_reset_envs, dim3(gx, m), dim3(256), 0, as_stream(stream), *b, ins ? *ins : none, from, ids);
+  }
   FFSRL_HIP(hipGetLastError());
   return 0;
 }

@@ -1062,20 +1062,47 @@ class SimModelDO:
         self.laparoscopeInCollision.zero_()
 
     # ------------------------------------------------------------------ reset
+    def _reset_in_one(self, ids) -> bool:
+        """Whether ``ffsrl_reset_envs`` can reset the environments ``ids``: all
+        of them in 0..numEnvs-1, on the current device, and every array the
+        batch's own (a caller may have put another in its place)."""
+        b, ins = self._batch, self._instrument
+        own = [(self.x, b.x), (self.p, b.p), (self.v, b.v), (self.drag, b.drag), (self.laparoscopeTip, b.tips),
+               (self.laparoscopeBase, b.caps_base)]
+        initial = [(self.initialVertex, self.x), (self.initialTips, self.laparoscopeTip),
+                   (self.initialBases, self.laparoscopeBase)]
+        if ins is not None:
+            own += [(self.laparoscopeXForm, ins.xform), (self.laparoscopeDragCutHeat, ins.drag_cut_heat),
+                    (self.laparoscopeDragCutHeatUpdate, ins.drag_cut_heat_update)]
+            initial.append((self.laparoscopeInitialXForm, self.laparoscopeXForm))
+        return (all(0 <= i < self.numEnvs for i in ids) and self.x.is_cuda
+                and self.x.device.index == torch.cuda.current_device()
+                and all(t.data_ptr() == p for t, p in own)
+                and all(t.is_contiguous() and t.dtype == torch.float32 and t.shape == u.shape and t.device == u.device
+                        for t, u in initial))
+
     def resetFixedModel(self, envNums):
         """``modelDO.py:1589-1622``: restore positions, zero predicted positions,
         velocities and grasp weights, restore the instrument points."""
-        for i in envNums:
-            s = self.env_slice(int(i))
+        ids = [int(i) for i in envNums]
+        if self._reset_in_one(ids):
+            arr = np.asarray(ids, np.int32)
+            ins = self._instrument
+            lib.ffsrl_reset_envs(self._batch, ins, _ptr(self.initialVertex), _ptr(self.initialTips),
+                                 _ptr(self.initialBases), None if ins is None else _ptr(self.laparoscopeInitialXForm),
+                                 arr.ctypes.data, len(ids), self.stream())
+            return
+        for i in ids:
+            s = self.env_slice(i)
             self.x[s] = self.initialVertex[s]
             self.p[s] = 0.0
             self.p[s, 3] = self.initialVertex[s, 3]
             self.v[s] = 0.0
             self.drag[s] = 0.0
-            self.laparoscopeTip[int(i)] = self.initialTips[int(i)]
-            self.laparoscopeBase[int(i)] = self.initialBases[int(i)]
+            self.laparoscopeTip[i] = self.initialTips[i]
+            self.laparoscopeBase[i] = self.initialBases[i]
             if self._instrument is not None:
-                k = int(i)
+                k = i
                 self.laparoscopeXForm[7 * k:7 * k + 7] = self.laparoscopeInitialXForm[7 * k:7 * k + 7]
                 self.laparoscopeDragCutHeat[3 * k:3 * k + 3] = 0
                 self.laparoscopeDragCutHeatUpdate[3 * k:3 * k + 3] = 0

@@ -432,6 +432,16 @@ int ffsrl_instrument_set_rcm(const ffsrl_batch* b, const ffsrl_instrument* ins, 
 /* updateLaparoscopeKernel (modelDO.py:218-245) alone. */
 int ffsrl_instrument_update(const ffsrl_batch* b, const ffsrl_instrument* ins, void* stream);
 
+/* Restores the n environments listed in envs (HOST memory; read before the
+ * call returns) to their initial state: positions and inverse masses from x0
+ * ([V*4], as x), predicted positions (0, 0, 0, w), velocities and grasp weights
+ * zero, the instrument points from tips0 / bases0 ([n_env*4*3]); with an
+ * instrument also its transforms from xform0 ([n_env*7*16]) and its clamp state
+ * zero.  ins NULL: the points only.  One launch per 500 environments, nothing
+ * allocated or copied.  Counterpart: resetFixedModel (modelDO.py:1589-1622). */
+int ffsrl_reset_envs(const ffsrl_batch* b, const ffsrl_instrument* ins, const float* x0, const float* tips0,
+                     const float* bases0, const float* xform0, const int32_t* envs, int32_t n, void* stream);
+
 /* ---- serving ------------------------------------------------------------ */
 
 /* Applies one tick of requests: a reset restores the env like resetFixedModel
