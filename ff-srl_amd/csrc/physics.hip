@@ -1347,11 +1347,19 @@ __global__ __launch_bounds__(BLOCK) void k_frame_shared(ffsrl_batch b, ffsrl_par
 // is claimed only by a running workgroup, after every part before it in the
 // order; so every env whose parts are all claimed completes, and its
 // workgroups then claim the next ones.  An env needs all its parts resident
-// at once: at most as many parts as the XCD has CUs (checked at launch), and
-// the launch should be the only persistent frame on the device (a partly
-// resident launch can leave an env's parts unclaimed until its waits give up,
-// which the frame reports as incomplete).  Waits are bounded as in the shared
-// frame; the last workgroup out checks, cleans up and resets every counter.
+// at once: at most as many parts as the XCD has CUs (checked at launch).
+//
+// Assembly: the parts of an env first wait for each other (parts_assemble),
+// before any of them touches the env's state.  Where other launches hold so
+// many CUs of the XCD that the parts of no env of this launch can come
+// together, the waiting parts withdraw from the env, and k_frame_rest, launched
+// behind the frame, runs it with one workgroup: the frame needs no
+// co-residency to complete.  Once assembled, an env's parts are all running
+// and its later waits end.  (An env above the one-workgroup frame's vertex
+// limit has no such form: there a partly
+// resident launch gives up and reports the frame as incomplete.)  Waits are
+// bounded as in the shared frame; the last workgroup out checks, cleans up and
+// resets every counter.
 struct PartsWs {
   const int32_t* parts;      // [n_parts][8]
   const int32_t* env_parts;  // int2 [n_env]
@@ -1361,14 +1369,16 @@ struct PartsWs {
   const uint64_t* f16;       // by part, its surface triangles' local ids (collision)
   unsigned long long* sums;  // [3][stride][2]
   int64_t stride;
-  uint32_t* ctr;             // [n_env][4]: parts finished, pass arrivals, give-up flag, 0; then XCD claim
-                             // counters [16], exits, and the claim table's first entry and size per XCD [16][2]
+  uint32_t* ctr;             // [n_env][4]: parts finished, pass arrivals, give-up flag, assembled parts | kWithdrawn;
+                             // then XCD claim counters [16], exits, workgroups at work per XCD [15], and the claim
+                             // table's first entry and size per XCD [16][2]
   int32_t* claims;           // per XCD, its parts in claim order: list slot << 6 | part
   int n_env;
   __device__ unsigned long long* plane(int k, int64_t vb) const { return sums + 2 * ((int64_t)k * stride + vb); }
   __device__ uint32_t* env_ctr(int env) const { return ctr + 4 * (int64_t)env; }
   __device__ uint32_t* xcd_ctr(int x) const { return ctr + 4 * (int64_t)n_env + x; }
   __device__ uint32_t* exits() const { return ctr + 4 * (int64_t)n_env + 16; }
+  __device__ uint32_t* working(int x) const { return ctr + 4 * (int64_t)n_env + 17 + x; }  // x < kWorkingXcds
   __device__ uint32_t* claim_info(int x) const { return ctr + 4 * (int64_t)n_env + 32 + 2 * x; }
 };
 
@@ -1774,6 +1784,38 @@ __device__ __forceinline__ void part_env(const ffsrl_batch& b, const ffsrl_param
   if (tid == 0 && sat_flag()) atomicOr(&b.status[env], (int32_t)FFSRL_STATUS_SATURATED);
 }
 
+// Set in an env's assembly word when its parts gave up waiting for each other:
+// k_frame_rest runs the env.
+constexpr uint32_t kWithdrawn = 1u << 31;
+constexpr int kWorkingXcds = 15;
+// Polls (of about a microsecond) without a workgroup of this launch at work on
+// the XCD after which a waiting part withdraws.  In a launch that has the device
+// to itself an env's missing parts are claimed as soon as workgroups finish
+// what they work on, so only a launch held back by others gets there.
+constexpr int kAssemblePolls = 1 << 11;
+
+// One thread of a part waits for the env's np parts to be claimed; false when
+// they withdraw from the env.  The first to give up sets kWithdrawn, and can only
+// while fewer than np have arrived; so either all np see np arrivals, or all see
+// the flag.
+__device__ __forceinline__ bool parts_assemble(uint32_t* word, uint32_t np, const uint32_t* working) {
+  uint32_t v = atomicAdd(word, 1u) + 1u;
+  int idle = 0;
+  for (int k = 0; !(v & kWithdrawn) && v < np; ++k) {
+    const bool none = working && __hip_atomic_load(working, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u;
+    idle = none ? idle + 1 : 0;
+    if (idle > kAssemblePolls || k >= kShareSpinLimit) {
+      const uint32_t seen = atomicCAS(word, v, v | kWithdrawn);
+      if (seen == v) return false;
+      v = seen;
+      continue;  // another part arrived or withdrew meanwhile
+    }
+    __builtin_amdgcn_s_sleep(2);
+    v = atomicAdd(word, 0u);
+  }
+  return !(v & kWithdrawn);
+}
+
 template <bool CARRY, bool COLLIDE>
 __global__ __launch_bounds__(1024) void k_frame_parts(ffsrl_batch b, ffsrl_params prm, const int32_t* list, int n,
                                                       int refit, int nxcd, XcdMap map, PartsWs ws) {
@@ -1795,11 +1837,21 @@ __global__ __launch_bounds__(1024) void k_frame_parts(ffsrl_batch b, ffsrl_param
       const int entry = ws.claims[c0 + k], el = entry >> 6, part = entry & 63;
       const int env = list ? list[el] : el;
       const int np = ws.env_parts[2 * env + 1];
+      uint32_t* working = x < kWorkingXcds ? ws.working(x) : nullptr;
+      if (np > 1) {
+        if (threadIdx.x == 0) s_claim = parts_assemble(&ws.env_ctr(env)[3], (uint32_t)np, working);
+        __syncthreads();
+        const bool go = __builtin_amdgcn_readfirstlane(s_claim) != 0;
+        __syncthreads();
+        if (!go) continue;
+      }
+      if (threadIdx.x == 0 && working) atomicAdd(working, 1u);
       if (np == 1)
         solo_env<CARRY, COLLIDE>(b, prm, ws, env, refit, lds);
       else
         part_env<CARRY, COLLIDE>(b, prm, ws, env, ws.env_parts[2 * env] + part, np, refit, lds);
       __syncthreads();  // LDS is reused by the next part
+      if (threadIdx.x == 0 && working) atomicSub(working, 1u);
     }
   }
   // The last workgroup out checks that every env's frame completed, clears
@@ -1816,8 +1868,11 @@ __global__ __launch_bounds__(1024) void k_frame_parts(ffsrl_batch b, ffsrl_param
   for (int el = threadIdx.x; el < n; el += 1024) {
     const int env = list ? list[el] : el;
     uint32_t* ctr = ws.env_ctr(env);
-    const bool inc =
-        atomicAdd(&ctr[0], 0u) != (uint32_t)ws.env_parts[2 * env + 1] || atomicAdd(&ctr[2], 0u) != 0u;
+    // a withdrawn env's state is as before the launch: its assembly word stays for k_frame_rest
+    const bool rest = (atomicAdd(&ctr[3], 0u) & kWithdrawn) != 0u && b.envs[env].nv <= kMaxFrameVertices;
+    const bool inc = !rest && (atomicAdd(&ctr[0], 0u) != (uint32_t)ws.env_parts[2 * env + 1] ||
+                               atomicAdd(&ctr[2], 0u) != 0u);
+    atomicExch(&ctr[3], rest ? kWithdrawn : 0u);
     if (inc) {
       atomicOr(&b.status[env], (int32_t)FFSRL_STATUS_INCOMPLETE);
       s_incomplete = 1;
@@ -1846,6 +1901,23 @@ __global__ __launch_bounds__(1024) void k_frame_parts(ffsrl_batch b, ffsrl_param
   __syncthreads();
   if (threadIdx.x < 16) atomicExch(ws.xcd_ctr(threadIdx.x), 0u);
   if (threadIdx.x == 0) atomicExch(ws.exits(), 0u);
+}
+
+// The envs whose parts withdrew (none in a launch that has the device to
+// itself: then every workgroup reads its envs' words and ends),
+// each by one workgroup as the one-workgroup frame.
+template <bool CARRY, bool COLLIDE>
+__global__ __launch_bounds__(1024) void k_frame_rest(ffsrl_batch b, ffsrl_params prm, const int32_t* list, int n,
+                                                     int refit, PartsWs ws) {
+  extern __shared__ unsigned long long lds[];
+  for (int el = blockIdx.x; el < n; el += gridDim.x) {
+    const int env = list ? list[el] : el;
+    uint32_t* word = &ws.env_ctr(env)[3];
+    if (!(*word & kWithdrawn)) continue;  // the same for every thread: written by the launch before
+    frame_env<1024, CARRY, COLLIDE>(b, prm, env, refit, lds);
+    __syncthreads();
+    if (threadIdx.x == 0) *word = 0u;
+  }
 }
 
 __global__ void k_xcc_probe(int32_t* out) {
@@ -2468,6 +2540,15 @@ int ffsrl_frame_parts(const ffsrl_batch* b, const ffsrl_params* prm, const ffsrl
   FFSRL_HIP(hipGetLastError());
   hipLaunchKernelGGL(kern, dim3(grid), dim3(1024), lds, st, *b, *prm, envs, n, refit, nxcd, map, ws);
   FFSRL_HIP(hipGetLastError());
+  if (pt->max_local > 0) {  // some env has several parts
+    auto rest = prm->collide ? (carry ? k_frame_rest<true, true> : k_frame_rest<false, true>)
+                             : (carry ? k_frame_rest<true, false> : k_frame_rest<false, false>);
+    const int rest_lds = lds_bytes_for(std::min(std::max(b->max_nv, 1), kMaxFrameVertices));
+    FFSRL_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(rest), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  rest_lds));
+    hipLaunchKernelGGL(rest, dim3(std::min(n, cus)), dim3(1024), rest_lds, st, *b, *prm, envs, n, refit, ws);
+    FFSRL_HIP(hipGetLastError());
+  }
   return 0;
 }
 

@@ -286,7 +286,7 @@ typedef struct ffsrl_parts {
   uint64_t* sums;                 /* [3][stride][2] fixed-point sums of shared vertices, by state
                                      vertex; zero before the first frame, left zero by every frame */
   int64_t stride;                 /* vertices per plane of sums (>= every env's vbase + nv) */
-  uint32_t* ctr;                  /* [4 n_env + 64]: counters in the first 4 n_env + 17 words (zero
+  uint32_t* ctr;                  /* [4 n_env + 64]: counters in the first 4 n_env + 32 words (zero
                                      before the first frame, left zero by every frame), then the
                                      claim table's extent per XCD (written by every launch) */
   int32_t* claims;                /* [n_claims] workspace: each launch's claim table */
@@ -303,11 +303,14 @@ typedef struct ffsrl_parts {
  * Jacobi sums), contact counts included; envs larger than the batched
  * frame's ffsrl_frame_max_vertices() run too, when their parts fit
  * (ffsrl_parts_max_local()).  All parts of an env run on one XCD at once:
- * at most CUs / XCDs (and 63) parts per env (FFSRL_E_LIMIT).  Two
- * launches: the claim table, then the frame.  The launch should be the
- * only persistent frame on the device: waits are bounded, and a frame that
- * could not complete sets FFSRL_STATUS_INCOMPLETE (its sums are cleared and
- * its counters reset).  envs NULL: environments 0 .. n-1.  Same reference
+ * at most CUs / XCDs (and 63) parts per env (FFSRL_E_LIMIT).  The
+ * launches are the claim table, the frame and, where an env has several
+ * parts, the one-workgroup frame of the envs whose parts could not come
+ * together because other launches held the XCD's CUs.  An env above
+ * ffsrl_frame_max_vertices() has no such form: for it the launch should be
+ * the only persistent frame on the device.  Waits are bounded, and a frame
+ * that could not complete sets FFSRL_STATUS_INCOMPLETE (its sums are cleared
+ * and its counters reset).  envs NULL: environments 0 .. n-1.  Same reference
  * counterpart as ffsrl_frame. */
 int ffsrl_frame_parts(const ffsrl_batch* b, const ffsrl_params* prm, const ffsrl_parts* parts,
                       const int32_t* envs, int32_t n, int32_t refit, void* stream);
