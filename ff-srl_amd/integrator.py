@@ -6,8 +6,13 @@ constraint projection with Jacobi averaging, the grasp pull and (with
 ``collision``) the instrument collision, the ground clamp and the integrate.
 Three launch forms run the same arithmetic:
 
-* batched (default): ``ffsrl_frame``, one launch for all environments and
-  the whole substep loop (and optionally the BVH refit);
+* batched (default): one launch for all environments and the whole substep
+  loop (and optionally the BVH refit), one workgroup per environment
+  (``ffsrl_frame``); a batch that would leave CUs idle that way runs in the
+  parts that ``SimModelDO.default_parts`` cuts instead, with the same bits.
+  One workgroup per environment is kept under stream capture, for a launch
+  shape other than the defaults or from the autotuner, and for a model with a
+  partition of its own;
 * shared (``shared=True``): ``ffsrl_frame_shared``, the same launch with all
   CUs sharing the environments (each env's frame cut into chunks that the
   workgroups of one XCD take in turn), for batches with fewer environments
@@ -37,6 +42,7 @@ class SimIntegratorDO:
         self.dispatch_sorted = dispatch_sorted
         self.shared = shared
         self.parts = parts
+        self.tuned = False  # a launch shape that the autotuner chose is kept
 
     def configure(self, cfg: dict) -> None:
         """Launch shape from the autotuner: {block, dispatch ("lpt"/"table"), shared, ...}."""
@@ -44,6 +50,7 @@ class SimIntegratorDO:
         self.dispatch_sorted = cfg["dispatch"] == "lpt"
         self.shared = bool(cfg.get("shared", False))
         self.parts = bool(cfg.get("parts", False))
+        self.tuned = True
 
     def autotune(self, simModel: SimModelDO, cache_path=None, frames: int = 2) -> dict:
         """Tune (or look up) the launch shape for this batch and use it."""
@@ -63,6 +70,9 @@ class SimIntegratorDO:
         elif self.shared:
             m.enable_shared()
             lib.ffsrl_frame_shared(m.batch, m.params, order, m.numEnvs, self.block, int(bool(refit)), m.stream())
+        elif (plan := m.default_parts() if self.block == 1024 and self.dispatch_sorted and not self.tuned
+              else None) is not None:
+            lib.ffsrl_frame_parts(m.batch, m.params, plan, order, m.numEnvs, int(bool(refit)), m.stream())
         else:
             lib.ffsrl_frame(m.batch, m.params, order, self.block, int(bool(refit)), m.stream())
 

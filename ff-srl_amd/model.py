@@ -18,8 +18,10 @@ from __future__ import annotations
 
 import concurrent.futures
 import ctypes as C
+import heapq
 import math
 import os
+from types import SimpleNamespace
 from typing import Optional, Sequence
 
 import numpy as np
@@ -97,6 +99,66 @@ def partition_mesh(tets: np.ndarray, edges: np.ndarray, nv: int, parts: int, use
     return {"rows": rows.astype(np.int64), "verts": verts[:n_verts.value], "tets16": t16[:nt].view(np.int64),
             "edges16": e16[:ne].view(np.int32), "tris16": f16[:nf].view(np.int64), "max_local": int(most.value),
             "parts": P}
+
+
+# Cost of a part of several beside its own constraints, in tets: the exchange of a
+# pass takes about 5 us on 64 ... 512 parts, a thousand tets about 3.4 us.
+EXCHANGE_TETS = 1500
+
+
+def default_tets_per_part(items, verts, env_mesh, cus: int, nxcd: int, collision: bool) -> Optional[int]:
+    """The partition of the default frame: the candidate whose longest CU is
+    estimated shortest, or None for one workgroup per env, which a partition
+    has to beat by a tenth.
+
+    items and verts: constraints (tets; edges without tet constraints) and
+    vertices of each mesh, env_mesh the mesh of each env.  With one workgroup
+    per env the frame lasts as long as its largest env, or as the fullest CU,
+    and the other CUs idle; parts fill them, but each part of several pays the
+    pass's exchange (with the collision pass a second, smaller one).  10 substeps of volume,
+    distance and Neo-Hookean, 1k-40k tets log-uniform, one workgroup per env
+    against 10,240 / 5,120 / 2,560 / 1,280 tets per part (us; * chosen):
+      16 envs 379: 330 221 151 123*      64 envs 1255: 411 278* 273 298
+      256 envs 1261: 623 602* 743 1043   512 envs 1268: 941* 1075 1346 1960
+      900 envs 1405*: 1589 1838 2322     with the collision pass 256 envs 1439: 762* 810 1072
+    20k-tet envs: 30 678: 327 276 213* 323; 300 1440: 1203 1191* 1636; 4k-tet envs:
+    120 183: - - 159* 216; 300 353*: - - 385 450."""
+    items, verts, env_mesh = (np.asarray(a, dtype=np.int64) for a in (items, verts, env_mesh))
+    if nxcd < 1 or env_mesh.size == 0:
+        return None
+    order = np.argsort(-items[env_mesh], kind="stable")
+    work = items[env_mesh][order]
+
+    def longest(costs, workers) -> int:
+        """Costs taken in order by whichever worker is free first."""
+        if len(costs) <= workers:
+            return int(max(costs, default=0))
+        free = [0] * workers
+        for c in costs:
+            heapq.heapreplace(free, free[0] + int(c))
+        return max(free)
+
+    if work.size > 8 * cus:  # as good as balanced: nothing to gain
+        return None
+    one = longest(work, cus)
+    if 10 * int(work.sum()) >= 9 * one * cus:
+        return None
+    per_xcd = min(cus // nxcd, PART_MAX)
+    cap, solo = int(lib.ffsrl_parts_max_local()), int(lib.ffsrl_parts_max_solo())
+    best, best_cost = None, 0.9 * one
+    for per in (1 << 30, 10240, 5120, 2560, 1280):
+        n = np.maximum(1, -(-items // per))
+        n = np.where((n == 1) & (verts > solo), 2, n)
+        n = np.where(n > 1, np.maximum(n, -(-verts * 5 // (4 * cap))), n)  # as _cut starts
+        if int(n.max(initial=1)) > per_xcd:
+            continue
+        cost = np.where(n > 1, -(-items // n) + EXCHANGE_TETS * (3 if collision else 2) // 2, items)
+        k = env_mesh[order]
+        t = max(longest(np.repeat(cost[k[x::nxcd]], n[k[x::nxcd]]), cus // nxcd) for x in range(nxcd))
+        if t < best_cost:
+            best, best_cost = per, t
+    return best
+
 
 _MODES = {None: OFF, "off": OFF, "pbd": PBD, "xpbd": XPBD}
 
@@ -406,6 +468,8 @@ class SimModelDO:
         if laparoscopes is not None:
             self._build_instrument(laps)
         self._order = None
+        self._default_store = self._default_built = self._default_modes = None
+        self._cut_default()
 
     @classmethod
     def from_usd(cls, path: str, numEnvs: int, device="cuda:0", **kw) -> "SimModelDO":
@@ -865,15 +929,9 @@ class SimModelDO:
         self._batch.fold_ws = _ptr(self.fold_ws)
         self._batch.fold_stride = self.numVertices if self.fold_ws is not None else 0
 
-    def enable_parts(self, tets_per_part: int = PART_TETS, parts: Optional[Sequence[int]] = None) -> Parts:
-        """Partition every mesh's constraints for the partitioned frame
-        (``ffsrl_frame_parts``) and allocate its sums and counters (zero, and
-        left at zero by every frame).  A mesh gets ceil(tets / tets_per_part)
-        parts (edges when the scheme has no tet constraints), more while a
-        part has more vertices than one workgroup's LDS holds (an env in one
-        part needs 32 B of LDS per vertex, a part of several 56 B); ``parts``
-        gives the count per mesh instead.  The partition follows the current
-        constraint order: ``set_constraint_order`` rebuilds it."""
+    def _cut(self, tets_per_part: int, parts: Optional[Sequence[int]] = None) -> list:
+        """The host part of a partition: ``partition_mesh`` of every mesh, with
+        the part counts of ``enable_parts``."""
         use_t = self.vol_mode != OFF or self.nh_on
         use_e = self.dist_mode != OFF
         cap = int(lib.ffsrl_parts_max_local())
@@ -901,7 +959,11 @@ class SimModelDO:
                                  f"{solo_cap if P == 1 else cap} that one workgroup holds ({P} parts)")
             return r
 
-        built = _parallel(build, range(len(self.topo)))
+        return _parallel(build, range(len(self.topo)))
+
+    def _upload_parts(self, store, built: list) -> Parts:
+        """The device part of a partition: its tables, sums and counters as
+        attributes of ``store``."""
         first = np.cumsum([0] + [r["parts"] for r in built])
         voff = np.cumsum([0] + [r["verts"].size for r in built])
         toff = np.cumsum([0] + [r["tris16"].size for r in built])
@@ -909,38 +971,96 @@ class SimModelDO:
         rows[:, 4] += np.repeat(voff[:-1], [r["parts"] for r in built])
         rows[:, 6] += np.repeat(toff[:-1], [r["parts"] for r in built])
         env_parts = np.stack([first[self.env_mesh], first[self.env_mesh + 1] - first[self.env_mesh]], axis=1)
-        self._parts_host = np.ascontiguousarray(env_parts.astype(np.int32))
+        store._parts_host = np.ascontiguousarray(env_parts.astype(np.int32))
         dev = self.device
         cat = np.concatenate
-        self.p_rows = torch.from_numpy(rows.astype(np.int32)).to(dev)
-        self.p_env = torch.from_numpy(self._parts_host).to(dev)
-        self.p_verts = torch.from_numpy(cat([r["verts"] for r in built])).to(dev)
-        self.p_tets16 = torch.from_numpy(cat([r["tets16"] for r in built])).to(dev)
-        self.p_edges16 = torch.from_numpy(cat([r["edges16"] for r in built])).to(dev)
+        store.p_rows = torch.from_numpy(rows.astype(np.int32)).to(dev)
+        store.p_env = torch.from_numpy(store._parts_host).to(dev)
+        store.p_verts = torch.from_numpy(cat([r["verts"] for r in built])).to(dev)
+        store.p_tets16 = torch.from_numpy(cat([r["tets16"] for r in built])).to(dev)
+        store.p_edges16 = torch.from_numpy(cat([r["edges16"] for r in built])).to(dev)
         # with the collision pass, the parts' triangles (one entry at least, so the table is never NULL)
-        self.p_tris16 = (torch.from_numpy(cat([r["tris16"] for r in built] + [np.zeros(1, np.int64)])).to(dev)
-                         if self.collision else None)
-        if getattr(self, "p_sums", None) is None:
-            self.p_sums = torch.zeros((3, self.numVertices, 2), dtype=torch.int64, device=dev)
-            self.p_ctr = torch.zeros(4 * self.numEnvs + 64, dtype=torch.int32, device=dev)
+        store.p_tris16 = (torch.from_numpy(cat([r["tris16"] for r in built] + [np.zeros(1, np.int64)])).to(dev)
+                          if self.collision else None)
+        if getattr(store, "p_sums", None) is None:
+            store.p_sums = torch.zeros((3, self.numVertices, 2), dtype=torch.int64, device=dev)
+            store.p_ctr = torch.zeros(4 * self.numEnvs + 64, dtype=torch.int32, device=dev)
             if lib.ffsrl_xcd_count() <= 0:
                 raise RuntimeError(f"ffsrl_xcd_count: {lib.ffsrl_last_error().decode()}")
         pt = Parts()
         pt.n_parts = int(rows.shape[0])
         pt.max_local = max([r["max_local"] for r in built if r["parts"] > 1], default=0)
         pt.max_solo = max([r["max_local"] for r in built if r["parts"] == 1], default=0)
-        pt.parts, pt.env_parts, pt.verts = _ptr(self.p_rows), _ptr(self.p_env), _ptr(self.p_verts)
-        pt.tets16, pt.edges16, pt.tris16 = _ptr(self.p_tets16), _ptr(self.p_edges16), _ptr(self.p_tris16)
-        pt.sums, pt.stride, pt.ctr = _ptr(self.p_sums), self.numVertices, _ptr(self.p_ctr)
-        n_claims = int(self._parts_host[:, 1].sum())
-        if getattr(self, "p_claims", None) is None or self.p_claims.numel() < n_claims:
-            self.p_claims = torch.zeros(n_claims, dtype=torch.int32, device=dev)
-        pt.claims, pt.n_claims = _ptr(self.p_claims), int(self.p_claims.numel())
-        pt.host_env_parts = self._parts_host.ctypes.data
+        pt.parts, pt.env_parts, pt.verts = _ptr(store.p_rows), _ptr(store.p_env), _ptr(store.p_verts)
+        pt.tets16, pt.edges16, pt.tris16 = _ptr(store.p_tets16), _ptr(store.p_edges16), _ptr(store.p_tris16)
+        pt.sums, pt.stride, pt.ctr = _ptr(store.p_sums), self.numVertices, _ptr(store.p_ctr)
+        n_claims = int(store._parts_host[:, 1].sum())
+        if getattr(store, "p_claims", None) is None or store.p_claims.numel() < n_claims:
+            store.p_claims = torch.zeros(n_claims, dtype=torch.int32, device=dev)
+        pt.claims, pt.n_claims = _ptr(store.p_claims), int(store.p_claims.numel())
+        pt.host_env_parts = store._parts_host.ctypes.data
+        return pt
+
+    def enable_parts(self, tets_per_part: int = PART_TETS, parts: Optional[Sequence[int]] = None) -> Parts:
+        """Partition every mesh's constraints for the partitioned frame
+        (``ffsrl_frame_parts``) and allocate its sums and counters (zero, and
+        left at zero by every frame).  A mesh gets ceil(tets / tets_per_part)
+        parts (edges when the scheme has no tet constraints), more while a
+        part has more vertices than one workgroup's LDS holds (an env in one
+        part needs 32 B of LDS per vertex, a part of several 56 B); ``parts``
+        gives the count per mesh instead.  The partition follows the current
+        constraint order: ``set_constraint_order`` rebuilds it."""
+        built = self._cut(tets_per_part, parts)
+        pt = self._upload_parts(self, built)
         self._parts = pt
         self._parts_cfg = dict(tets_per_part=tets_per_part, parts=parts)
         self.parts_per_mesh = [r["parts"] for r in built]
         return pt
+
+    def _default_tets_per_part(self) -> Optional[int]:
+        """Tets per part of the default frame's own partition, or None where
+        the default frame keeps one workgroup per env (``ffsrl_frame``), by
+        the longest CU of each (``default_tets_per_part``)."""
+        if not self.x.is_cuda or self.numVertices == 0 or self.max_nv > int(lib.ffsrl_frame_max_vertices()):
+            return None
+        use_t = self.vol_mode != OFF or self.nh_on
+        items = [m.num_tets if use_t else m.num_edges for m in self.meshes]
+        cus = torch.cuda.get_device_properties(self.x.device).multi_processor_count
+        return default_tets_per_part(items, [m.num_vertices for m in self.meshes], self.env_mesh, cus,
+                                     int(lib.ffsrl_xcd_count()), self.collision)
+
+    def _cut_default(self) -> None:
+        """(Re)cut the default frame's partition; its tables are uploaded by the
+        first frame that uses them."""
+        if self._default_store is not None:
+            torch.cuda.synchronize(self.device)  # frames in flight on any stream read the tables
+        self._default_store = self._default_built = None
+        self._default_modes = (self.vol_mode != OFF or self.nh_on, self.dist_mode != OFF, self.collision)
+        per_part = self._default_tets_per_part()
+        if per_part is None:
+            return
+        try:
+            built = self._cut(per_part)
+        except ValueError:  # a mesh that its parts cannot hold: one workgroup per env
+            return
+        nxcd = int(lib.ffsrl_xcd_count())
+        cus = torch.cuda.get_device_properties(self.x.device).multi_processor_count
+        if nxcd > 0 and max(r["parts"] for r in built) <= min(cus // nxcd, PART_MAX):
+            self._default_built = built
+
+    def default_parts(self) -> Optional[Parts]:
+        """The partition that ``SimIntegratorDO``'s default frame uses (None: one
+        workgroup per env).  It is separate from ``enable_parts``'s; a model
+        that has one of its own keeps one workgroup per env as its default."""
+        if getattr(self, "_parts", None) is not None or torch.cuda.is_current_stream_capturing():
+            return None
+        if self._default_modes != (self.vol_mode != OFF or self.nh_on, self.dist_mode != OFF, self.collision):
+            self._cut_default()
+        if self._default_built is not None:
+            store = SimpleNamespace()
+            store.pt = self._upload_parts(store, self._default_built)
+            self._default_store, self._default_built = store, None
+        return None if self._default_store is None else self._default_store.pt
 
     @property
     def parts(self) -> Parts:
@@ -1011,6 +1131,7 @@ class SimModelDO:
         self.constraint_order = constraint_order
         if getattr(self, "_parts", None) is not None:
             self.enable_parts(**self._parts_cfg)   # the partition follows the constraint order
+        self._default_modes = None                 # and so does the default frame's, cut again by its next frame
 
     def dispatch_order(self) -> torch.Tensor:
         """Environments largest first: the hardware dispatcher then assigns
