@@ -1026,8 +1026,17 @@ class SimModelDO:
         use_t = self.vol_mode != OFF or self.nh_on
         items = [m.num_tets if use_t else m.num_edges for m in self.meshes]
         cus = torch.cuda.get_device_properties(self.x.device).multi_processor_count
-        return default_tets_per_part(items, [m.num_vertices for m in self.meshes], self.env_mesh, cus,
-                                     int(lib.ffsrl_xcd_count()), self.collision)
+        per = default_tets_per_part(items, [m.num_vertices for m in self.meshes], self.env_mesh, cus,
+                                    int(lib.ffsrl_xcd_count()), self.collision)
+        # A full chip, each env in one part: its positions in LDS instead of global memory.  Faster with
+        # Neo-Hookean, whose inverse rest matrices fill the caches (us, one workgroup per env / one part:
+        # 20k tets x 1024 envs, one iteration 3146 / 2931, two 7081 / 6204; 1.5k x 256 105 / 103), except with
+        # collision and two iterations (7831 / 8240, registers); slower without (volume and distance 2356 / 2572)
+        # and on an idle chip (4k x 4 168 / 171: the claim table's launch).
+        if (per is None and self.nh_on and self.numEnvs >= cus and not (self.collision and self.simConstraints > 1)
+                and self.max_nv <= int(lib.ffsrl_parts_max_solo())):
+            return 1 << 30
+        return per
 
     def _cut_default(self) -> None:
         """(Re)cut the default frame's partition; its tables are uploaded by the

@@ -128,3 +128,22 @@ def test_what_keeps_one_workgroup_per_env(pkg, gpu):
     assert big.max_nv > pkg.lib.ffsrl_frame_max_vertices() and big.default_parts() is None
     with pytest.raises(pkg.FFSRLError, match="ffsrl_frame failed"):
         pkg.SimIntegratorDO(gpu).stepModel(big)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("collision,iterations,parts", [(False, 1, True), (False, 2, True), (True, 1, True), (True, 2, False)])
+def test_full_chip_of_whole_envs(pkg, gpu, collision, iterations, parts):
+    """At least as many Neo-Hookean envs as CUs, each within one part's LDS."""
+    n = torch.cuda.get_device_properties(gpu).multi_processor_count
+    n += -n % 8
+    mesh = pkg.scenes.solid("box", 600, seed=3)
+    tip = np.repeat((pkg.scenes.top_point(mesh) + np.array([0.0, 0.02, 0.0], np.float32))[None], 4, axis=0)
+    kw = dict(BASE, distance="xpbd", volume="xpbd", neoHookean=True, simConstraintsSteps=iterations,
+              tips=np.tile(tip[None], (n, 1, 1)).astype(np.float32))
+    if collision:
+        kw.update(collision=True, globalKsContact=1.0, capsuleBases=kw["tips"] + np.array([0.0, 0.5, 0.0], np.float32),
+                  capsuleRadii=np.full((n, 4), 0.03, np.float32))
+    a, b = (pkg.SimModelDO([mesh], [0] * n, device=gpu, **kw) for _ in range(2))
+    pt = b.default_parts()
+    assert (pt is not None) == parts and (pt is None or pt.max_local == 0)
+    _frames(pkg, gpu, a, b)
