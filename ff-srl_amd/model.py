@@ -469,7 +469,7 @@ class SimModelDO:
             self._build_instrument(laps)
         self._order = None
         self._default_store = self._default_built = self._default_modes = None
-        self._cut_default()
+        self.default_parts()   # cut and uploaded here, not by the first frame
 
     @classmethod
     def from_usd(cls, path: str, numEnvs: int, device="cuda:0", **kw) -> "SimModelDO":
@@ -1013,6 +1013,9 @@ class SimModelDO:
         built = self._cut(tets_per_part, parts)
         pt = self._upload_parts(self, built)
         self._parts = pt
+        if self._default_store is not None:    # not used any more (default_parts)
+            torch.cuda.synchronize(self.device)
+            self._default_store = None
         self._parts_cfg = dict(tets_per_part=tets_per_part, parts=parts)
         self.parts_per_mesh = [r["parts"] for r in built]
         return pt
@@ -1039,8 +1042,7 @@ class SimModelDO:
         return per
 
     def _cut_default(self) -> None:
-        """(Re)cut the default frame's partition; its tables are uploaded by the
-        first frame that uses them."""
+        """(Re)cut the default frame's partition."""
         if self._default_store is not None:
             torch.cuda.synchronize(self.device)  # frames in flight on any stream read the tables
         self._default_store = self._default_built = None
@@ -1061,7 +1063,7 @@ class SimModelDO:
         """The partition that ``SimIntegratorDO``'s default frame uses (None: one
         workgroup per env).  It is separate from ``enable_parts``'s; a model
         that has one of its own keeps one workgroup per env as its default."""
-        if getattr(self, "_parts", None) is not None or torch.cuda.is_current_stream_capturing():
+        if getattr(self, "_parts", None) is not None or not self.x.is_cuda or torch.cuda.is_current_stream_capturing():
             return None
         if self._default_modes != (self.vol_mode != OFF or self.nh_on, self.dist_mode != OFF, self.collision):
             self._cut_default()

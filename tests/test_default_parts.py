@@ -104,7 +104,6 @@ def test_what_keeps_one_workgroup_per_env(pkg, gpu):
     with torch.cuda.graph(g, stream=s):
         assert b.default_parts() is None
         pkg.SimIntegratorDO(gpu).stepModel(b, refit=True)
-    assert b._default_store is None
     for _ in range(3):
         pkg.lib.ffsrl_frame(a.batch, a.params, a.dispatch_order().data_ptr(), 1024, 1, a.stream())
         g.replay()
@@ -121,9 +120,9 @@ def test_what_keeps_one_workgroup_per_env(pkg, gpu):
     tuned = pkg.SimIntegratorDO(gpu)
     tuned.configure({"block": 1024, "dispatch": "lpt"})
     tuned.stepModel(b)
-    assert b._default_store is None
+    assert b._default_store is not None
     b.enable_parts()
-    assert b.default_parts() is None
+    assert b.default_parts() is None and b._default_store is None
     big = pkg.SimModelDO([pkg.scenes.cube_grid(23)], [0], device=gpu, distance="pbd", volume="pbd")
     assert big.max_nv > pkg.lib.ffsrl_frame_max_vertices() and big.default_parts() is None
     with pytest.raises(pkg.FFSRLError, match="ffsrl_frame failed"):
