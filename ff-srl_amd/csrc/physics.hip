@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "constraints.hpp"
+#include "parts_wait.hpp"
 #include "refit.hpp"
 
 namespace ffsrl {
@@ -1356,10 +1357,10 @@ __global__ __launch_bounds__(BLOCK) void k_frame_shared(ffsrl_batch b, ffsrl_par
 // behind the frame, runs it with one workgroup: the frame needs no
 // co-residency to complete.  Once assembled, an env's parts are all running
 // and its later waits end.  (An env above the one-workgroup frame's vertex
-// limit has no such form: there a partly
-// resident launch gives up and reports the frame as incomplete.)  Waits are
-// bounded as in the shared frame; the last workgroup out checks, cleans up and
-// resets every counter.
+// limit has no such form: its parts wait until the CUs are free, and only a
+// launch that stays partly resident for kShareSpinLimit polls gives up and
+// reports the frame as incomplete.)  Waits are bounded as in the shared frame;
+// the last workgroup out checks, cleans up and resets every counter.
 struct PartsWs {
   const int32_t* parts;      // [n_parts][8]
   const int32_t* env_parts;  // int2 [n_env]
@@ -1784,37 +1785,26 @@ __device__ __forceinline__ void part_env(const ffsrl_batch& b, const ffsrl_param
   if (tid == 0 && sat_flag()) atomicOr(&b.status[env], (int32_t)FFSRL_STATUS_SATURATED);
 }
 
-// Set in an env's assembly word when its parts gave up waiting for each other:
-// k_frame_rest runs the env.
-constexpr uint32_t kWithdrawn = 1u << 31;
 constexpr int kWorkingXcds = 15;
 // Polls (of about a microsecond) without a workgroup of this launch at work on
-// the XCD after which a waiting part withdraws.  In a launch that has the device
-// to itself an env's missing parts are claimed as soon as workgroups finish
-// what they work on, so only a launch held back by others gets there.
+// the XCD after which the parts of an env that k_frame_rest can run withdraw.
+// In a launch that has the device to itself an env's missing parts are claimed
+// as soon as workgroups finish what they work on, so only a launch held back by
+// others gets there.  The parts of a larger env wait as long as share_wait does:
+// another stream's kernel may hold the CUs for longer than that.
 constexpr int kAssemblePolls = 1 << 11;
 
-// One thread of a part waits for the env's np parts to be claimed; false when
-// they withdraw from the env.  The first to give up sets kWithdrawn, and can only
-// while fewer than np have arrived; so either all np see np arrivals, or all see
-// the flag.
-__device__ __forceinline__ bool parts_assemble(uint32_t* word, uint32_t np, const uint32_t* working) {
-  uint32_t v = atomicAdd(word, 1u) + 1u;
-  int idle = 0;
-  for (int k = 0; !(v & kWithdrawn) && v < np; ++k) {
-    const bool none = working && __hip_atomic_load(working, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u;
-    idle = none ? idle + 1 : 0;
-    if (idle > kAssemblePolls || k >= kShareSpinLimit) {
-      const uint32_t seen = atomicCAS(word, v, v | kWithdrawn);
-      if (seen == v) return false;
-      v = seen;
-      continue;  // another part arrived or withdrew meanwhile
-    }
-    __builtin_amdgcn_s_sleep(2);
-    v = atomicAdd(word, 0u);
+// An env's assembly word (parts_wait.hpp), and the workgroups at work on the XCD.
+struct AssemblyWord {
+  uint32_t* word;
+  const uint32_t* working;
+  __device__ uint32_t add(uint32_t n) { return atomicAdd(word, n); }
+  __device__ uint32_t cas(uint32_t expected, uint32_t desired) { return atomicCAS(word, expected, desired); }
+  __device__ bool idle() {
+    return working && __hip_atomic_load(working, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u;
   }
-  return !(v & kWithdrawn);
-}
+  __device__ void pause() { __builtin_amdgcn_s_sleep(2); }
+};
 
 template <bool CARRY, bool COLLIDE>
 __global__ __launch_bounds__(1024) void k_frame_parts(ffsrl_batch b, ffsrl_params prm, const int32_t* list, int n,
@@ -1839,7 +1829,9 @@ __global__ __launch_bounds__(1024) void k_frame_parts(ffsrl_batch b, ffsrl_param
       const int np = ws.env_parts[2 * env + 1];
       uint32_t* working = x < kWorkingXcds ? ws.working(x) : nullptr;
       if (np > 1) {
-        if (threadIdx.x == 0) s_claim = parts_assemble(&ws.env_ctr(env)[3], (uint32_t)np, working);
+        if (threadIdx.x == 0)
+          s_claim = parts_assemble(AssemblyWord{&ws.env_ctr(env)[3], working}, (uint32_t)np,
+                                   b.envs[env].nv <= kMaxFrameVertices ? kAssemblePolls : 0, kShareSpinLimit);
         __syncthreads();
         const bool go = __builtin_amdgcn_readfirstlane(s_claim) != 0;
         __syncthreads();

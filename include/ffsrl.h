@@ -307,8 +307,8 @@ typedef struct ffsrl_parts {
  * launches are the claim table, the frame and, where an env has several
  * parts, the one-workgroup frame of the envs whose parts could not come
  * together because other launches held the XCD's CUs.  An env above
- * ffsrl_frame_max_vertices() has no such form: for it the launch should be
- * the only persistent frame on the device.  Waits are bounded, and a frame
+ * ffsrl_frame_max_vertices() has no such form: its parts wait for the CUs, and
+ * the launch should be the only persistent frame on the device.  Waits are bounded, and a frame
  * that could not complete sets FFSRL_STATUS_INCOMPLETE (its sums are cleared
  * and its counters reset).  envs NULL: environments 0 .. n-1.  Same reference
  * counterpart as ffsrl_frame. */
