@@ -20,20 +20,23 @@ constexpr uint32_t kWithdrawn = 1u << 31;
 // waits do, whatever else holds the CUs).
 //
 // Word: add(n) and cas(expected, desired) return the word before, idle()
-// whether no workgroup is at work, pause() passes the time between polls.
+// whether no workgroup is at work (asked every kIdleEvery polls), pause(k) passes
+// the time after the k-th poll.
+constexpr int kIdleEvery = 8;
+
 template <class Word>
-__host__ __device__ inline bool parts_assemble(Word&& word, uint32_t np, int idle_polls, int polls) {
+__host__ __device__ inline bool parts_assemble(Word word, uint32_t np, int idle_polls, int polls) {
   uint32_t v = word.add(1u) + 1u;
   int idle = 0;
-  for (int k = 0; !(v & kWithdrawn) && v < np; ++k) {
-    idle = idle_polls && word.idle() ? idle + 1 : 0;
-    if (idle > idle_polls || k >= polls) {
+  for (int k = 1; !(v & kWithdrawn) && v < np; ++k) {
+    if (idle_polls && k % kIdleEvery == 0) idle = word.idle() ? idle + kIdleEvery : 0;
+    if (idle > idle_polls || k > polls) {
       const uint32_t seen = word.cas(v, v | kWithdrawn);
       if (seen == v) return false;
       v = seen;
       continue;  // another part arrived or withdrew meanwhile
     }
-    word.pause();
+    word.pause(k);
     v = word.add(0u);
   }
   return !(v & kWithdrawn);

@@ -1371,15 +1371,14 @@ struct PartsWs {
   unsigned long long* sums;  // [3][stride][2]
   int64_t stride;
   uint32_t* ctr;             // [n_env][4]: parts finished, pass arrivals, give-up flag, assembled parts | kWithdrawn;
-                             // then XCD claim counters [16], exits, workgroups at work per XCD [15], and the claim
-                             // table's first entry and size per XCD [16][2]
-  int32_t* claims;           // per XCD, its parts in claim order: list slot << 6 | part
+                             // then XCD claim counters [16], exits, 15 spare, and the claim table's first entry and
+                             // size per XCD [16][2]
+  int32_t* claims;           // per XCD, its parts in claim order: env << 6 | part
   int n_env;
   __device__ unsigned long long* plane(int k, int64_t vb) const { return sums + 2 * ((int64_t)k * stride + vb); }
   __device__ uint32_t* env_ctr(int env) const { return ctr + 4 * (int64_t)env; }
   __device__ uint32_t* xcd_ctr(int x) const { return ctr + 4 * (int64_t)n_env + x; }
   __device__ uint32_t* exits() const { return ctr + 4 * (int64_t)n_env + 16; }
-  __device__ uint32_t* working(int x) const { return ctr + 4 * (int64_t)n_env + 17 + x; }  // x < kWorkingXcds
   __device__ uint32_t* claim_info(int x) const { return ctr + 4 * (int64_t)n_env + 32 + 2 * x; }
 };
 
@@ -1394,10 +1393,11 @@ __global__ __launch_bounds__(1024) void k_parts_claims(const int32_t* list, int 
   __shared__ int count[16], first[16];
   const int lane = threadIdx.x & 63, x = threadIdx.x >> 6;
   const int cnt = x < nxcd && x < n ? (n - 1 - x) / nxcd + 1 : 0;  // slots of XCD x
-  auto parts_of = [&](int j) { return j < cnt ? ws.env_parts[2 * (list ? list[x + nxcd * j] : x + nxcd * j) + 1] : 0; };
+  auto env_of = [&](int j) { return j >= cnt ? -1 : list ? list[x + nxcd * j] : x + nxcd * j; };
+  auto parts_of = [&](int env) { return env >= 0 ? ws.env_parts[2 * env + 1] : 0; };
   int total = 0;
   for (int j0 = 0; j0 < cnt; j0 += 64) {
-    int v = parts_of(j0 + lane);
+    int v = parts_of(env_of(j0 + lane));
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
     total += v;
   }
@@ -1414,14 +1414,13 @@ __global__ __launch_bounds__(1024) void k_parts_claims(const int32_t* list, int 
   if (x >= nxcd) return;
   int base = first[x];
   for (int j0 = 0; j0 < cnt; j0 += 64) {
-    const int j = j0 + lane, np = parts_of(j);
+    const int env = env_of(j0 + lane), np = parts_of(env);
     int incl = np;
     for (int off = 1; off < 64; off <<= 1) {
       const int t = __shfl_up(incl, off);
       if (lane >= off) incl += t;
     }
-    const int el = x + nxcd * j;
-    for (int q = 0; q < np; ++q) ws.claims[base + incl - np + q] = (el << 6) | q;
+    for (int q = 0; q < np; ++q) ws.claims[base + incl - np + q] = (env << 6) | q;
     base += __shfl(incl, 63);
   }
   if (lane == 0) {
@@ -1566,6 +1565,54 @@ __device__ __forceinline__ void solo_env(const ffsrl_batch& b, const ffsrl_param
   }
   __syncthreads();
   if (refit) refit_env<BLOCK>(b, e);
+}
+
+// Polls (of about a microsecond) without a workgroup of this launch at work on
+// the XCD after which the parts of an env that k_frame_rest can run withdraw.
+// In a launch that has the device to itself an env's missing parts are claimed
+// as soon as workgroups finish what they work on, so only a launch held back by
+// others gets there.  The parts of a larger env wait as long as share_wait does:
+// another stream's kernel may hold the CUs for longer than that.
+constexpr int kAssemblePolls = 1 << 11;
+
+// The assembly word (parts_wait.hpp) of an env.  Claims are in slot order, so
+// every part of the envs of the XCD's earlier claims has been claimed, and of
+// later envs none while a part of this one has not: a workgroup is at work where
+// the env of an earlier claim is neither finished nor withdrawn.  (Counts of the
+// workgroups at work, kept by every part on neighbouring words, cost 9 us a
+// frame on 64 envs of 6,000 tets, 5 parts each: one substep 64.5 -> 55.9 us.)
+struct AssemblyWord {
+  uint32_t* ctr;
+  const int32_t* env_parts;
+  const int32_t* claims;  // the XCD's first that may be at work
+  uint32_t* word;
+  __device__ uint32_t add(uint32_t n) { return atomicAdd(word, n); }
+  __device__ uint32_t cas(uint32_t expected, uint32_t desired) { return atomicCAS(word, expected, desired); }
+  __device__ bool idle() {  // one claim further with each call
+    const int env = *claims >> 6;
+    uint32_t* c = ctr + 4 * (int64_t)env;
+    if (&c[3] == word) return true;
+    if (atomicAdd(&c[0], 0u) >= (uint32_t)env_parts[2 * env + 1] || (atomicAdd(&c[3], 0u) & kWithdrawn)) ++claims;
+    return false;
+  }
+  // After the first polls the wait is for workgroups to come free: fewer polls
+  // beside their exchanges' own, on the same lines.
+  __device__ void pause(int k) {
+    if (k < 16)
+      __builtin_amdgcn_s_sleep(2);
+    else
+      __builtin_amdgcn_s_sleep(48);
+  }
+};
+
+// v in vector registers from here on.  One thread's operands, computed where it
+// waits: in scalar registers the compiler computes them ahead of the claim loop and
+// keeps them across the frames, where they push the projection's constants out
+// (256 mixed scenes with two iterations 1005 -> 1110 us).
+template <class T>
+__device__ __forceinline__ T in_vector(T v) {
+  asm volatile("" : "+v"(v));
+  return v;
 }
 
 // A part of a multi-part env.  Each pass (projection; with COLLIDE also the
@@ -1785,27 +1832,6 @@ __device__ __forceinline__ void part_env(const ffsrl_batch& b, const ffsrl_param
   if (tid == 0 && sat_flag()) atomicOr(&b.status[env], (int32_t)FFSRL_STATUS_SATURATED);
 }
 
-constexpr int kWorkingXcds = 15;
-// Polls (of about a microsecond) without a workgroup of this launch at work on
-// the XCD after which the parts of an env that k_frame_rest can run withdraw.
-// In a launch that has the device to itself an env's missing parts are claimed
-// as soon as workgroups finish what they work on, so only a launch held back by
-// others gets there.  The parts of a larger env wait as long as share_wait does:
-// another stream's kernel may hold the CUs for longer than that.
-constexpr int kAssemblePolls = 1 << 11;
-
-// An env's assembly word (parts_wait.hpp), and the workgroups at work on the XCD.
-struct AssemblyWord {
-  uint32_t* word;
-  const uint32_t* working;
-  __device__ uint32_t add(uint32_t n) { return atomicAdd(word, n); }
-  __device__ uint32_t cas(uint32_t expected, uint32_t desired) { return atomicCAS(word, expected, desired); }
-  __device__ bool idle() {
-    return working && __hip_atomic_load(working, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u;
-  }
-  __device__ void pause() { __builtin_amdgcn_s_sleep(2); }
-};
-
 template <bool CARRY, bool COLLIDE>
 __global__ __launch_bounds__(1024) void k_frame_parts(ffsrl_batch b, ffsrl_params prm, const int32_t* list, int n,
                                                       int refit, int nxcd, XcdMap map, PartsWs ws) {
@@ -1824,31 +1850,32 @@ __global__ __launch_bounds__(1024) void k_frame_parts(ffsrl_batch b, ffsrl_param
       __syncthreads();  // s_claim is written again by the next claim
       if (k >= cn) break;
       // the k-th part of this XCD's slots x, x + nxcd, ... in order
-      const int entry = ws.claims[c0 + k], el = entry >> 6, part = entry & 63;
-      const int env = list ? list[el] : el;
+      const int entry = ws.claims[c0 + k], env = entry >> 6, part = entry & 63;
       const int np = ws.env_parts[2 * env + 1];
-      uint32_t* working = x < kWorkingXcds ? ws.working(x) : nullptr;
       if (np > 1) {
-        if (threadIdx.x == 0)
-          s_claim = parts_assemble(AssemblyWord{&ws.env_ctr(env)[3], working}, (uint32_t)np,
+        if (threadIdx.x == 0) {
+          uint32_t* ctr = in_vector(ws.ctr);
+          const AssemblyWord word{ctr, in_vector(ws.env_parts), in_vector(ws.claims) + in_vector(c0),
+                                  ctr + 4 * (int64_t)in_vector(env) + 3};
+          s_claim = parts_assemble(word, (uint32_t)in_vector(np),
                                    b.envs[env].nv <= kMaxFrameVertices ? kAssemblePolls : 0, kShareSpinLimit);
+        }
         __syncthreads();
         const bool go = __builtin_amdgcn_readfirstlane(s_claim) != 0;
         __syncthreads();
         if (!go) continue;
       }
-      if (threadIdx.x == 0 && working) atomicAdd(working, 1u);
       if (np == 1)
         solo_env<CARRY, COLLIDE>(b, prm, ws, env, refit, lds);
       else
         part_env<CARRY, COLLIDE>(b, prm, ws, env, ws.env_parts[2 * env] + part, np, refit, lds);
       __syncthreads();  // LDS is reused by the next part
-      if (threadIdx.x == 0 && working) atomicSub(working, 1u);
     }
   }
   // The last workgroup out checks that every env's frame completed, clears
   // the planes of any that did not (a part that gave up leaves partial
   // sums), reports it, and resets the counters for the next launch.
+  wait_vmem();  // this workgroup's counts are in before it is counted out
   __syncthreads();
   if (threadIdx.x == 0) s_lastwg = atomicAdd(ws.exits(), 1u) == gridDim.x - 1;
   __syncthreads();
@@ -1860,10 +1887,10 @@ __global__ __launch_bounds__(1024) void k_frame_parts(ffsrl_batch b, ffsrl_param
   for (int el = threadIdx.x; el < n; el += 1024) {
     const int env = list ? list[el] : el;
     uint32_t* ctr = ws.env_ctr(env);
-    // a withdrawn env's state is as before the launch: its assembly word stays for k_frame_rest
-    const bool rest = (atomicAdd(&ctr[3], 0u) & kWithdrawn) != 0u && b.envs[env].nv <= kMaxFrameVertices;
-    const bool inc = !rest && (atomicAdd(&ctr[0], 0u) != (uint32_t)ws.env_parts[2 * env + 1] ||
-                               atomicAdd(&ctr[2], 0u) != 0u);
+    const uint32_t finished = atomicAdd(&ctr[0], 0u), gave_up = atomicAdd(&ctr[2], 0u), word = atomicAdd(&ctr[3], 0u);
+    // a withdrawn env's state is as before the launch; its assembly word stays for k_frame_rest
+    const bool rest = (word & kWithdrawn) != 0u && b.envs[env].nv <= kMaxFrameVertices;
+    const bool inc = !rest && (finished != (uint32_t)ws.env_parts[2 * env + 1] || gave_up != 0u);
     atomicExch(&ctr[3], rest ? kWithdrawn : 0u);
     if (inc) {
       atomicOr(&b.status[env], (int32_t)FFSRL_STATUS_INCOMPLETE);
@@ -2504,7 +2531,7 @@ int ffsrl_frame_parts(const ffsrl_batch* b, const ffsrl_params* prm, const ffsrl
   }
   if (total > pt->n_claims) return fail(FFSRL_E_ARG, "parts: %lld claim entries for %lld parts", (long long)pt->n_claims,
                                         (long long)total);
-  if (n >= (1 << 25)) return fail(FFSRL_E_LIMIT, "%d environments listed (claim entries hold 2^25)", n);
+  if (b->n_env >= (1 << 25)) return fail(FFSRL_E_LIMIT, "%d environments (claim entries hold 2^25)", b->n_env);
   const int lds = std::max(kPartLocalBytes * pt->max_local, kSoloBytes * pt->max_solo);
   auto kern = prm->collide ? (carry ? k_frame_parts<true, true> : k_frame_parts<false, true>)
                            : (carry ? k_frame_parts<true, false> : k_frame_parts<false, false>);

@@ -24,7 +24,7 @@ struct Word {
     return expected;
   }
   bool idle() { return working->load() == 0; }
-  void pause() {
+  void pause(int) {
     polls->fetch_add(1);
     std::this_thread::yield();
   }
