@@ -101,18 +101,24 @@ def partition_mesh(tets: np.ndarray, edges: np.ndarray, nv: int, parts: int, use
             "parts": P}
 
 
-# Cost of a part of several beside its own constraints, in tets: the exchange of a
-# pass takes about 5 us on 64 ... 512 parts, a thousand tets about 3.4 us.
+# Costs beside the constraints themselves, in tets (a thousand take about 2.5 us):
+# of a pass of one workgroup, and of a pass of a part of several (the exchange,
+# about 5 us on 64 ... 512 parts); once a frame, the start and end of an env or
+# part of several, and the partitioned frame's two more launches.
+PASS_TETS = 400
 EXCHANGE_TETS = 1500
+ENV_TETS, PART_START_TETS, FRAME_TETS = 2400, 4000, 2400
 
 
-def default_tets_per_part(items, verts, env_mesh, cus: int, nxcd: int, collision: bool) -> Optional[int]:
+def default_tets_per_part(items, verts, env_mesh, cus: int, nxcd: int, collision: bool,
+                          passes: int = 10) -> Optional[int]:
     """The partition of the default frame: the candidate whose longest CU is
     estimated shortest, or None for one workgroup per env, which a partition
-    has to beat by a tenth.
+    has to beat by 8%.
 
     items and verts: constraints (tets; edges without tet constraints) and
-    vertices of each mesh, env_mesh the mesh of each env.  With one workgroup
+    vertices of each mesh, env_mesh the mesh of each env, passes the frame's
+    substeps times iterations.  With one workgroup
     per env the frame lasts as long as its largest env, or as the fullest CU,
     and the other CUs idle; parts fill them, but each part of several pays the
     pass's exchange (with the collision pass a second, smaller one).  10 substeps of volume,
@@ -122,12 +128,17 @@ def default_tets_per_part(items, verts, env_mesh, cus: int, nxcd: int, collision
       256 envs 1261: 623 602* 743 1043   512 envs 1268: 941* 1075 1346 1960
       900 envs 1405*: 1589 1838 2322     with the collision pass 256 envs 1439: 762* 810 1072
     20k-tet envs: 30 678: 327 276 213* 323; 300 1440: 1203 1191* 1636; 4k-tet envs:
-    120 183: - - 159* 216; 300 353*: - - 385 450."""
+    120 183: - - 159* 216; 300 353*: - - 385 450.
+    A frame of few passes also pays for the parts' start and the launches (volume and
+    distance, one workgroup per env / parts, by substeps): 4k tets, 1 env: 1 18* / 24, 2 29* / 30,
+    4 51 / 41*, 30 envs: 2 30* / 33, 4 53 / 45*, 100 envs: 4 55* / 59, 8 100 / 94*; 9k, 100 envs:
+    1 36* / 38, 2 58 / 53*; 500 mixed envs: 1 80* / 94, 2 142* / 152."""
     items, verts, env_mesh = (np.asarray(a, dtype=np.int64) for a in (items, verts, env_mesh))
     if nxcd < 1 or env_mesh.size == 0:
         return None
+    whole = passes * (items + PASS_TETS) + ENV_TETS
     order = np.argsort(-items[env_mesh], kind="stable")
-    work = items[env_mesh][order]
+    work = whole[env_mesh][order]
 
     def longest(costs, workers) -> int:
         """Costs taken in order by whichever worker is free first."""
@@ -141,20 +152,21 @@ def default_tets_per_part(items, verts, env_mesh, cus: int, nxcd: int, collision
     if work.size > 8 * cus:  # as good as balanced: nothing to gain
         return None
     one = longest(work, cus)
-    if 10 * int(work.sum()) >= 9 * one * cus:
+    if 100 * int(work.sum()) >= 92 * one * cus:
         return None
     per_xcd = min(cus // nxcd, PART_MAX)
     cap, solo = int(lib.ffsrl_parts_max_local()), int(lib.ffsrl_parts_max_solo())
-    best, best_cost = None, 0.9 * one
+    best, best_cost = None, 0.92 * one
     for per in (1 << 30, 10240, 5120, 2560, 1280):
         n = np.maximum(1, -(-items // per))
         n = np.where((n == 1) & (verts > solo), 2, n)
         n = np.where(n > 1, np.maximum(n, -(-verts * 5 // (4 * cap))), n)  # as _cut starts
         if int(n.max(initial=1)) > per_xcd:
             continue
-        cost = np.where(n > 1, -(-items // n) + EXCHANGE_TETS * (3 if collision else 2) // 2, items)
+        exchange = EXCHANGE_TETS * (3 if collision else 2) // 2
+        cost = np.where(n > 1, passes * (-(-items // n) + exchange) + PART_START_TETS, whole)
         k = env_mesh[order]
-        t = max(longest(np.repeat(cost[k[x::nxcd]], n[k[x::nxcd]]), cus // nxcd) for x in range(nxcd))
+        t = max(longest(np.repeat(cost[k[x::nxcd]], n[k[x::nxcd]]), cus // nxcd) for x in range(nxcd)) + FRAME_TETS
         if t < best_cost:
             best, best_cost = per, t
     return best
@@ -1030,7 +1042,7 @@ class SimModelDO:
         items = [m.num_tets if use_t else m.num_edges for m in self.meshes]
         cus = torch.cuda.get_device_properties(self.x.device).multi_processor_count
         per = default_tets_per_part(items, [m.num_vertices for m in self.meshes], self.env_mesh, cus,
-                                    int(lib.ffsrl_xcd_count()), self.collision)
+                                    int(lib.ffsrl_xcd_count()), self.collision, self.simSubsteps * self.simConstraints)
         # A full chip, each env in one part: its positions in LDS instead of global memory.  Faster with
         # Neo-Hookean, whose inverse rest matrices fill the caches (us, one workgroup per env / one part:
         # 20k tets x 1024 envs, one iteration 3146 / 2931, two 7081 / 6204; 1.5k x 256 105 / 103), except with

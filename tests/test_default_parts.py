@@ -146,3 +146,17 @@ def test_full_chip_of_whole_envs(pkg, gpu, collision, iterations, parts):
     pt = b.default_parts()
     assert (pt is not None) == parts and (pt is None or pt.max_local == 0)
     _frames(pkg, gpu, a, b)
+
+
+@pytest.mark.parametrize("items,env_mesh,passes,parts", [
+    ([4000], [0], 1, False), ([4000], [0], 2, False), ([4000], [0], 4, True),
+    ([4000], [0] * 100, 2, False), ([4000], [0] * 100, 4, False), ([4000], [0] * 100, 8, True),
+    ([6000], [0] * 30, 1, False), ([6000], [0] * 100, 2, False), ([6000], [0] * 100, 4, True),
+    ([9000], [0] * 100, 1, False), ([9000], [0] * 100, 2, True), ([20000], [0] * 100, 1, False),
+    ([20000], [0], 1, True), ([20000], [0] * 30, 1, True), ([30000, 12000, 5000, 2000], [0, 1, 2, 3] * 125, 1, False),
+])
+def test_rule_few_passes(pkg, items, env_mesh, passes, parts):
+    """Parts start and end once a frame: a frame of few passes must win that back."""
+    import importlib
+    f = importlib.import_module("ff-srl_amd.model").default_tets_per_part
+    assert (f(items, [t // 4 for t in items], env_mesh, 256, 8, False, passes) is not None) == parts
