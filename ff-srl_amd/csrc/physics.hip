@@ -1449,7 +1449,7 @@ constexpr int kSoloMaxVertices = (kLdsBytes - kPartStaticLds) / kSoloBytes;
 // weights stay in the model's arrays as there.  Each pass has no exchange and
 // no wait; the model's p is written once, after the last pass.
 template <bool CARRY, bool COLLIDE>
-__device__ __forceinline__ void solo_env(const ffsrl_batch& b, const ffsrl_params& prm, const PartsWs& ws, int env, int refit,
+__device__ __forceinline__ void solo_env(const ffsrl_batch& b, const ffsrl_params& prm, uint32_t* finished, int env, int refit,
                          unsigned long long* lds) {
   constexpr int BLOCK = 1024;
   const ffsrl_env_desc e = b.envs[env];
@@ -1560,7 +1560,7 @@ __device__ __forceinline__ void solo_env(const ffsrl_batch& b, const ffsrl_param
   for (int i = tid; i < nv; i += BLOCK) st4(b.p, vb + i, Pl[i]);
   if (tid == 0) {
     if (COLLIDE && s_contacts) atomicAdd(&b.in_collision[env], s_contacts);  // counts accumulate until cleared
-    atomicAdd(&ws.env_ctr(env)[0], 1u);  // the env's one part is done
+    if (finished) atomicAdd(finished, 1u);  // the env's one part is done
     if (sat_flag()) atomicOr(&b.status[env], (int32_t)FFSRL_STATUS_SATURATED);
   }
   __syncthreads();
@@ -1866,7 +1866,7 @@ __global__ __launch_bounds__(1024) void k_frame_parts(ffsrl_batch b, ffsrl_param
         if (!go) continue;
       }
       if (np == 1)
-        solo_env<CARRY, COLLIDE>(b, prm, ws, env, refit, lds);
+        solo_env<CARRY, COLLIDE>(b, prm, ws.env_ctr(env), env, refit, lds);
       else
         part_env<CARRY, COLLIDE>(b, prm, ws, env, ws.env_parts[2 * env] + part, np, refit, lds);
       __syncthreads();  // LDS is reused by the next part
@@ -1920,6 +1920,17 @@ __global__ __launch_bounds__(1024) void k_frame_parts(ffsrl_batch b, ffsrl_param
   __syncthreads();
   if (threadIdx.x < 16) atomicExch(ws.xcd_ctr(threadIdx.x), 0u);
   if (threadIdx.x == 0) atomicExch(ws.exits(), 0u);
+}
+
+// Every env in one part: one workgroup each, as k_frame with solo_env's form, and
+// no claims, waits or counters.  Neo-Hookean envs, volume and distance, no refit (us:
+// k_frame / claimed as above / here): 256 of 600 tets, one substep 15.5 / 18.4 /
+// 10.4, ten 50 / 53.5 / 44.4; 1,024 of 5,000, one 104 / 108 / 98, ten 741 / 742 / 733.
+template <bool CARRY, bool COLLIDE>
+__global__ __launch_bounds__(1024) void k_frame_solo(ffsrl_batch b, ffsrl_params prm, const int32_t* list, int refit) {
+  extern __shared__ float4 lds_parts[];
+  solo_env<CARRY, COLLIDE>(b, prm, nullptr, list ? list[blockIdx.x] : (int)blockIdx.x, refit,
+                           reinterpret_cast<unsigned long long*>(lds_parts));
 }
 
 // The envs whose parts withdrew (none in a launch that has the device to
@@ -2513,9 +2524,11 @@ int ffsrl_frame_parts(const ffsrl_batch* b, const ffsrl_params* prm, const ffsrl
   }
   const int per_xcd = std::min(cus / nxcd, 63);
   int64_t total = 0;
+  bool several = false;  // some env has several parts
   for (int i = 0; i < b->n_env; ++i) {
     const int np = pt->host_env_parts[2 * i + 1];
     total += np;
+    several |= np > 1;
     if (np < 1 || np > per_xcd)
       return fail(FFSRL_E_LIMIT, "env %d has %d parts; they must run at once on one XCD (%d CUs)", i, np, per_xcd);
     if (b->host_envs) {
@@ -2532,6 +2545,16 @@ int ffsrl_frame_parts(const ffsrl_batch* b, const ffsrl_params* prm, const ffsrl
   if (total > pt->n_claims) return fail(FFSRL_E_ARG, "parts: %lld claim entries for %lld parts", (long long)pt->n_claims,
                                         (long long)total);
   if (b->n_env >= (1 << 25)) return fail(FFSRL_E_LIMIT, "%d environments (claim entries hold 2^25)", b->n_env);
+  hipStream_t st = as_stream(stream);
+  if (!several) {
+    const int lds = kSoloBytes * pt->max_solo;
+    auto solo = prm->collide ? (carry ? k_frame_solo<true, true> : k_frame_solo<false, true>)
+                             : (carry ? k_frame_solo<true, false> : k_frame_solo<false, false>);
+    FFSRL_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(solo), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    hipLaunchKernelGGL(solo, dim3(n), dim3(1024), lds, st, *b, *prm, envs, refit);
+    FFSRL_HIP(hipGetLastError());
+    return 0;
+  }
   const int lds = std::max(kPartLocalBytes * pt->max_local, kSoloBytes * pt->max_solo);
   auto kern = prm->collide ? (carry ? k_frame_parts<true, true> : k_frame_parts<false, true>)
                            : (carry ? k_frame_parts<true, false> : k_frame_parts<false, false>);
@@ -2554,20 +2577,17 @@ int ffsrl_frame_parts(const ffsrl_batch* b, const ffsrl_params* prm, const ffsrl
                    pt->ctr,
                    pt->claims,
                    b->n_env};
-  hipStream_t st = as_stream(stream);
   hipLaunchKernelGGL(k_parts_claims, dim3(1), dim3(1024), 0, st, envs, n, nxcd, ws);
   FFSRL_HIP(hipGetLastError());
   hipLaunchKernelGGL(kern, dim3(grid), dim3(1024), lds, st, *b, *prm, envs, n, refit, nxcd, map, ws);
   FFSRL_HIP(hipGetLastError());
-  if (pt->max_local > 0) {  // some env has several parts
-    auto rest = prm->collide ? (carry ? k_frame_rest<true, true> : k_frame_rest<false, true>)
-                             : (carry ? k_frame_rest<true, false> : k_frame_rest<false, false>);
-    const int rest_lds = lds_bytes_for(std::min(std::max(b->max_nv, 1), kMaxFrameVertices));
-    FFSRL_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(rest), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  rest_lds));
-    hipLaunchKernelGGL(rest, dim3(std::min(n, cus)), dim3(1024), rest_lds, st, *b, *prm, envs, n, refit, ws);
-    FFSRL_HIP(hipGetLastError());
-  }
+  auto rest = prm->collide ? (carry ? k_frame_rest<true, true> : k_frame_rest<false, true>)
+                           : (carry ? k_frame_rest<true, false> : k_frame_rest<false, false>);
+  const int rest_lds = lds_bytes_for(std::min(std::max(b->max_nv, 1), kMaxFrameVertices));
+  FFSRL_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(rest), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                rest_lds));
+  hipLaunchKernelGGL(rest, dim3(std::min(n, cus)), dim3(1024), rest_lds, st, *b, *prm, envs, n, refit, ws);
+  FFSRL_HIP(hipGetLastError());
   return 0;
 }
 

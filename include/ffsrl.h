@@ -304,9 +304,9 @@ typedef struct ffsrl_parts {
  * frame's ffsrl_frame_max_vertices() run too, when their parts fit
  * (ffsrl_parts_max_local()).  All parts of an env run on one XCD at once:
  * at most CUs / XCDs (and 63) parts per env (FFSRL_E_LIMIT).  The
- * launches are the claim table, the frame and, where an env has several
- * parts, the one-workgroup frame of the envs whose parts could not come
- * together because other launches held the XCD's CUs.  An env above
+ * launches are the claim table, the frame and the one-workgroup frame of the
+ * envs whose parts could not come together because other launches held the
+ * XCD's CUs; a batch with every env in one part takes one launch.  An env above
  * ffsrl_frame_max_vertices() has no such form: its parts wait for the CUs, and
  * the launch should be the only persistent frame on the device.  Waits are bounded, and a frame
  * that could not complete sets FFSRL_STATUS_INCOMPLETE (its sums are cleared

@@ -31,3 +31,36 @@ def test_two_models_on_two_streams(pkg, gpu, tets, envs):
     for a, b in zip(ref, got):
         assert int(b.frame_status().abs().sum()) == 0
         assert all(torch.equal(getattr(a, k), getattr(b, k)) for k in ("x", "v", "p", "bvh_lo", "bvh_hi"))
+
+
+@pytest.mark.parametrize("mode", ["nh", "xpbd", "collision"])
+@pytest.mark.parametrize("listed", [False, True])
+def test_every_env_in_one_part(pkg, gpu, mode, listed):
+    """Envs of one part each, listed or not, at the largest size and the smallest."""
+    sc = pkg.scenes
+    meshes = [sc.solid("ellipsoid", 20000, seed=81), sc.solid("box", 40, seed=82), sc.solid("box", 2000, seed=83)]
+    assert pkg.lib.ffsrl_parts_max_solo() - 64 < meshes[0].num_vertices <= pkg.lib.ffsrl_parts_max_solo()
+    kw = dict(simSubsteps=3, simConstraintsSteps=2, distance="xpbd", volume="xpbd", neoHookean=mode == "nh")
+    if mode == "collision":
+        low = torch.stack([torch.from_numpy(sc.top_point(m)) for m in meshes for _ in range(4)]).reshape(3, 4, 3).float()
+        low[..., 1] -= 0.036
+        low = low.repeat(3, 1, 1)
+        kw.update(collision=True, globalKsContact=1.0, capsuleBases=low.numpy(), tips=(low + torch.tensor([0.0, 0.62, 0.0])).numpy(),
+                  capsuleRadii=torch.tensor([0.12, 0, 0, 0]).repeat(9, 1).numpy())
+    a, b = (pkg.SimModelDO(meshes, [0, 1, 2] * 3, device=gpu, **kw) for _ in range(2))
+    b.enable_parts(tets_per_part=1 << 30)
+    assert b.parts.max_local == 0
+    order = torch.tensor([7, 0, 4, 8, 3], dtype=torch.int32, device=gpu) if listed else None
+    for _ in range(3):
+        if listed:
+            pkg.lib.ffsrl_frame_envs(a.batch, a.params, order.data_ptr(), 5, 1024, 1, a.stream())
+            pkg.lib.ffsrl_frame_parts(b.batch, b.params, b.parts, order.data_ptr(), 5, 1, b.stream())
+        else:
+            pkg.lib.ffsrl_frame(a.batch, a.params, None, 1024, 1, a.stream())
+            pkg.lib.ffsrl_frame_parts(b.batch, b.params, b.parts, None, 9, 1, b.stream())
+    torch.cuda.synchronize()
+    for k in ("x", "v", "p", "bvh_lo", "bvh_hi", "status", "laparoscopeInCollision", "lam_t", "lam_e"):
+        s, t = getattr(a, k), getattr(b, k)
+        assert (s is None and t is None) or torch.equal(s, t), k
+    if mode == "collision":
+        assert int(a.laparoscopeInCollision.sum()) > 0
