@@ -99,6 +99,7 @@ class RaycastRendererDO:
         self.rot_q = q
         self.dirs = torch.from_numpy(ray_directions(self.height, self.width, q, self.v_aperture,
                                                     self.h_aperture)).to(self.device)
+        self._dirs_made = None if self.dirs.is_inference() else self.dirs._version
         cam = Camera()
         cam.origin[:] = tuple(float(c) for c in self.cameraPos.astype(np.float32))
         cam.dirs = self.dirs.data_ptr()
@@ -141,11 +142,36 @@ class RaycastRendererDO:
         self.camera.mode = int(render_mode)
 
     def set_traversal(self, traversal: int) -> None:
-        """0: a wavefront walks the BVH for a block of rays (the default), 1
-        one ray per lane, 2 a lane per pixel's 2x2 rays.  The images are the
-        same bit for bit."""
+        """0: a wavefront walks the BVH for a block of rays (the default; with
+        directions that a caller has put into the table, the faster of the other
+        two), 1 one ray per lane, 2 a lane per pixel's 2x2 rays.  The images are
+        the same bit for bit."""
         self.traversal = int(traversal)
         self.camera.traversal = self.traversal
+
+    def _traversal(self, n: int) -> int:
+        """The traversal of ``n`` environments.  The block form is for the table
+        of a pinhole, as the renderer makes it; it traces the rays of any other one
+        by one at a lower occupancy than the other two forms.  128x128 depth of a
+        fisheye, 4k- and 20k-tet scenes, block / per ray / quads (us): 8 envs
+        65 / 63 / 135, 64 (16,384 blocks of 8x8 pixels) 346 / 232 / 274, 256
+        1,122 / 856 / 792; 64x64, 256 envs 447 / 287 / 337."""
+        cam = self.camera
+        own = cam.dirs == self.dirs.data_ptr() and (self._dirs_made is None or self._dirs_made == self.dirs._version)
+        if cam.traversal or own:
+            return cam.traversal
+        blocks = n * -(-cam.width // 8) * -(-cam.height // 8)
+        return 2 if cam.width * cam.height >= 128 * 128 and blocks >= 32768 else 1
+
+    def _camera(self, n: int, mode: int) -> Camera:
+        """The camera, or a copy of it, for a call in ``mode`` over ``n`` environments."""
+        traversal = self._traversal(n)
+        if self.camera.mode == mode and self.camera.traversal == traversal:
+            return self.camera
+        cam = Camera()
+        C.pointer(cam)[0] = self.camera
+        cam.mode, cam.traversal = mode, traversal
+        return cam
 
     def depth_camera(self) -> Camera:
         """A copy of the camera in depth mode (the renderer keeps its mode)."""
@@ -157,7 +183,7 @@ class RaycastRendererDO:
     def render_depth(self, env_begin: int = 0, env_end: int = None, hit=None, thit=None) -> torch.Tensor:
         m = self.simModel
         ee = m.numEnvs if env_end is None else env_end
-        cam = self.camera if self.camera.mode == RenderMode.depth_map else self.depth_camera()
+        cam = self._camera(ee - env_begin, RenderMode.depth_map)
         out = self.depth[env_begin:ee]
         lib.ffsrl_render(m.batch, cam, env_begin, ee, out.data_ptr(), None, None, None, None,
                          None if hit is None else hit.data_ptr(), None if thit is None else thit.data_ptr(),
@@ -171,7 +197,8 @@ class RaycastRendererDO:
             raise ValueError("render_rgb needs a colour render mode")
         lib.ffsrl_vertex_normals(m.batch, env_begin, ee, m.normals.data_ptr(), m.stream())
         out = self.pixels[env_begin:ee]
-        lib.ffsrl_render(m.batch, self.camera, env_begin, ee, None, out.data_ptr(), m.normals.data_ptr(),
+        cam = self._camera(ee - env_begin, self.camera.mode)
+        lib.ffsrl_render(m.batch, cam, env_begin, ee, None, out.data_ptr(), m.normals.data_ptr(),
                          m.vertexColors.data_ptr(), m.t_tri_colors.data_ptr(), None, None, m.stream())
         return out
 
@@ -184,7 +211,8 @@ class RaycastRendererDO:
             raise ValueError("render_rgbd needs a colour render mode")
         lib.ffsrl_vertex_normals(m.batch, env_begin, ee, m.normals.data_ptr(), m.stream())
         pix, dep = self.pixels[env_begin:ee], self.depth[env_begin:ee]
-        lib.ffsrl_render(m.batch, self.camera, env_begin, ee, dep.data_ptr(), pix.data_ptr(), m.normals.data_ptr(),
+        cam = self._camera(ee - env_begin, self.camera.mode)
+        lib.ffsrl_render(m.batch, cam, env_begin, ee, dep.data_ptr(), pix.data_ptr(), m.normals.data_ptr(),
                          m.vertexColors.data_ptr(), m.t_tri_colors.data_ptr(), None, None, m.stream())
         return pix, dep
 

@@ -181,7 +181,7 @@ typedef struct ffsrl_camera {
  * colours bit for bit; they differ only in speed.  AUTO: a wavefront walks the
  * BVH once for a block of rays (8x8 to 16x16, by the size of the launch); it is
  * fastest for a pinhole table of directions, and traces the rays of any other
- * one by one.  PER_RAY: a lane traces one supersampled ray.  QUAD: a lane
+ * one by one, slower than PER_RAY or, for large images, QUAD.  PER_RAY: a lane traces one supersampled ray.  QUAD: a lane
  * traces the 2x2 rays of its pixel with one stack (a BVH of at most 2^28 - 1
  * nodes, which AUTO asks for too from 128x128 output pixels). */
 #define FFSRL_TRAVERSE_AUTO 0
