@@ -321,7 +321,7 @@ class SceneServer:
                 lib.ffsrl_frame_shared(model.batch, model.params, p_step, m, self.block, 1, s)
             elif m:
                 lib.ffsrl_frame_envs(model.batch, model.params, p_step, m, self.block, 1, s)
-            cam = self.renderer.camera
+            cam = self.renderer._camera(n, self.renderer.camera.mode)
             lib.ffsrl_render_envs(model.batch, cam, p_env, n, self.depth.data_ptr(), None, None, None, None, None,
                                   None, s)
             lib.ffsrl_observe_envs(model.batch, p_env, n, self.x0.data_ptr(), float(model.groundLevel),
