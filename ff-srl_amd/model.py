@@ -941,11 +941,16 @@ class SimModelDO:
         self._batch.fold_ws = _ptr(self.fold_ws)
         self._batch.fold_stride = self.numVertices if self.fold_ws is not None else 0
 
+    def _modes(self) -> tuple:
+        """Whether a frame with the parameters as they are (a caller may have set
+        them since) projects tets and edges and runs the collision pass."""
+        p = self.params
+        return bool(p.vol_mode != OFF or p.nh_on), p.dist_mode != OFF, bool(p.collide)
+
     def _cut(self, tets_per_part: int, parts: Optional[Sequence[int]] = None) -> list:
         """The host part of a partition: ``partition_mesh`` of every mesh, with
         the part counts of ``enable_parts``."""
-        use_t = self.vol_mode != OFF or self.nh_on
-        use_e = self.dist_mode != OFF
+        use_t, use_e, collide = self._modes()
         cap = int(lib.ffsrl_parts_max_local())
         solo_cap = int(lib.ffsrl_parts_max_solo())
 
@@ -961,7 +966,7 @@ class SimModelDO:
                 P = max(P, min(PART_MAX, -(-m.num_vertices * 5 // (4 * cap))))
             while True:
                 r = partition_mesh(t.tets, t.edges, m.num_vertices, P, use_t, use_e,
-                                   tris=t.tris_leaf if self.collision else None)
+                                   tris=t.tris_leaf if collide else None)
                 limit = solo_cap if P == 1 else cap
                 if r["max_local"] <= limit or parts is not None or P >= PART_MAX:
                     break
@@ -993,7 +998,7 @@ class SimModelDO:
         store.p_edges16 = torch.from_numpy(cat([r["edges16"] for r in built])).to(dev)
         # with the collision pass, the parts' triangles (one entry at least, so the table is never NULL)
         store.p_tris16 = (torch.from_numpy(cat([r["tris16"] for r in built] + [np.zeros(1, np.int64)])).to(dev)
-                          if self.collision else None)
+                          if self.params.collide else None)
         if getattr(store, "p_sums", None) is None:
             store.p_sums = torch.zeros((3, self.numVertices, 2), dtype=torch.int64, device=dev)
             store.p_ctr = torch.zeros(4 * self.numEnvs + 64, dtype=torch.int32, device=dev)
@@ -1038,17 +1043,18 @@ class SimModelDO:
         the longest CU of each (``default_tets_per_part``)."""
         if not self.x.is_cuda or self.numVertices == 0 or self.max_nv > int(lib.ffsrl_frame_max_vertices()):
             return None
-        use_t = self.vol_mode != OFF or self.nh_on
+        use_t, _, collide = self._modes()
+        p = self.params
         items = [m.num_tets if use_t else m.num_edges for m in self.meshes]
         cus = torch.cuda.get_device_properties(self.x.device).multi_processor_count
         per = default_tets_per_part(items, [m.num_vertices for m in self.meshes], self.env_mesh, cus,
-                                    int(lib.ffsrl_xcd_count()), self.collision, self.simSubsteps * self.simConstraints)
+                                    int(lib.ffsrl_xcd_count()), collide, p.substeps * p.iterations)
         # A full chip, each env in one part: its positions in LDS instead of global memory.  Faster with
         # Neo-Hookean, whose inverse rest matrices fill the caches (us, one workgroup per env / one part:
         # 20k tets x 1024 envs, one iteration 3146 / 2931, two 7081 / 6204; 1.5k x 256 105 / 103), except with
         # collision and two iterations (7831 / 8240, registers); slower without (volume and distance 2356 / 2572)
         # and on an idle chip (4k x 4 168 / 171: the claim table's launch).
-        if (per is None and self.nh_on and self.numEnvs >= cus and not (self.collision and self.simConstraints > 1)
+        if (per is None and p.nh_on and self.numEnvs >= cus and not (collide and p.iterations > 1)
                 and self.max_nv <= int(lib.ffsrl_parts_max_solo())):
             return 1 << 30
         return per
@@ -1058,7 +1064,7 @@ class SimModelDO:
         if self._default_store is not None:
             torch.cuda.synchronize(self.device)  # frames in flight on any stream read the tables
         self._default_store = self._default_built = None
-        self._default_modes = (self.vol_mode != OFF or self.nh_on, self.dist_mode != OFF, self.collision)
+        self._default_modes = self._modes()
         per_part = self._default_tets_per_part()
         if per_part is None:
             return
@@ -1077,7 +1083,7 @@ class SimModelDO:
         that has one of its own keeps one workgroup per env as its default."""
         if getattr(self, "_parts", None) is not None or not self.x.is_cuda or torch.cuda.is_current_stream_capturing():
             return None
-        if self._default_modes != (self.vol_mode != OFF or self.nh_on, self.dist_mode != OFF, self.collision):
+        if self._default_modes != self._modes():
             self._cut_default()
         if self._default_built is not None:
             store = SimpleNamespace()
