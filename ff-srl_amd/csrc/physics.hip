@@ -1898,7 +1898,7 @@ __global__ __launch_bounds__(1024) void k_frame_parts(ffsrl_batch b, ffsrl_param
     }
     atomicExch(&ctr[0], 0u);
     atomicExch(&ctr[1], 0u);
-    atomicExch(&ctr[2], inc ? 2u : 0u);
+    atomicExch(&ctr[2], inc && ws.env_parts[2 * env + 1] > 1 ? 2u : 0u);  // an env in one part has no sums
   }
   __syncthreads();
   if (s_incomplete) {
@@ -2538,7 +2538,7 @@ int ffsrl_frame_parts(const ffsrl_batch* b, const ffsrl_params* prm, const ffsrl
       if (h.max_terms > FFSRL_MAX_TERMS)
         return fail(FFSRL_E_LIMIT, "env %d: a vertex receives %d Jacobi terms in one pass (limit %d)", i,
                     h.max_terms, FFSRL_MAX_TERMS);
-      if ((int64_t)h.vbase + h.nv > pt->stride)
+      if (np > 1 && (int64_t)h.vbase + h.nv > pt->stride)  // an env in one part has no sums here
         return fail(FFSRL_E_ARG, "parts stride %lld < vbase + nv of env %d", (long long)pt->stride, i);
     }
   }

@@ -410,13 +410,17 @@ class SimModelDO:
                  constraint_order: str = "local", globalKsContact=1.0, collision: bool = False,
                  capsuleBases: Optional[np.ndarray] = None, capsuleRadii: Optional[np.ndarray] = None,
                  laparoscopes=None, workspaceLow=(-1e5, -1e5, -1e5), workspaceHigh=(1e5, 1e5, 1e5),
-                 bvh_on_device: bool = False):
+                 bvh_on_device: bool = False, default_partition: bool = True):
         """``meshes`` and ``env_mesh``: the simulated meshes and each env's
         mesh.  The reference's form ``SimModelDO(stage, numEnvs, device, ...)``
         (``modelDO.py:774``) is accepted too: a USD crate scene path (or its
         converted ``.npz``), or an opened stage (its root layer's file), and
         the number of envs; every env then holds the scene's meshes and
-        laparoscope (``self.scene`` keeps the parsed scene)."""
+        laparoscope (``self.scene`` keeps the parsed scene).
+
+        ``default_partition=False`` leaves the default frame's partition
+        (``default_parts``) to the first frame that uses it, for a model that is
+        driven otherwise."""
         self.scene = None
         if isinstance(meshes, (str, os.PathLike)) or hasattr(meshes, "GetRootLayer"):
             from .usd_scene import merged_mesh, scene
@@ -480,8 +484,9 @@ class SimModelDO:
         if laparoscopes is not None:
             self._build_instrument(laps)
         self._order = None
-        self._default_store = self._default_built = self._default_modes = None
-        self.default_parts()   # cut and uploaded here, not by the first frame
+        self._default_store = self._default_modes = None
+        if default_partition:
+            self.default_parts()   # cut and uploaded here, not by the first frame
 
     @classmethod
     def from_usd(cls, path: str, numEnvs: int, device="cuda:0", **kw) -> "SimModelDO":
@@ -999,8 +1004,12 @@ class SimModelDO:
         # with the collision pass, the parts' triangles (one entry at least, so the table is never NULL)
         store.p_tris16 = (torch.from_numpy(cat([r["tris16"] for r in built] + [np.zeros(1, np.int64)])).to(dev)
                           if self.params.collide else None)
-        if getattr(store, "p_sums", None) is None:
-            store.p_sums = torch.zeros((3, self.numVertices, 2), dtype=torch.int64, device=dev)
+        # an env in one part exchanges no sums
+        summed = self.numVertices if any(r["parts"] > 1 for r in built) else 1
+        if getattr(store, "p_sums", None) is None or store.p_sums.shape[1] < summed:
+            store.p_sums = None
+            store.p_sums = torch.zeros((3, summed, 2), dtype=torch.int64, device=dev)
+        if getattr(store, "p_ctr", None) is None:
             store.p_ctr = torch.zeros(4 * self.numEnvs + 64, dtype=torch.int32, device=dev)
             if lib.ffsrl_xcd_count() <= 0:
                 raise RuntimeError(f"ffsrl_xcd_count: {lib.ffsrl_last_error().decode()}")
@@ -1010,7 +1019,7 @@ class SimModelDO:
         pt.max_solo = max([r["max_local"] for r in built if r["parts"] == 1], default=0)
         pt.parts, pt.env_parts, pt.verts = _ptr(store.p_rows), _ptr(store.p_env), _ptr(store.p_verts)
         pt.tets16, pt.edges16, pt.tris16 = _ptr(store.p_tets16), _ptr(store.p_edges16), _ptr(store.p_tris16)
-        pt.sums, pt.stride, pt.ctr = _ptr(store.p_sums), self.numVertices, _ptr(store.p_ctr)
+        pt.sums, pt.stride, pt.ctr = _ptr(store.p_sums), int(store.p_sums.shape[1]), _ptr(store.p_ctr)
         n_claims = int(store._parts_host[:, 1].sum())
         if getattr(store, "p_claims", None) is None or store.p_claims.numel() < n_claims:
             store.p_claims = torch.zeros(n_claims, dtype=torch.int32, device=dev)
@@ -1028,11 +1037,11 @@ class SimModelDO:
         gives the count per mesh instead.  The partition follows the current
         constraint order: ``set_constraint_order`` rebuilds it."""
         built = self._cut(tets_per_part, parts)
-        pt = self._upload_parts(self, built)
-        self._parts = pt
         if self._default_store is not None:    # not used any more (default_parts)
             torch.cuda.synchronize(self.device)
             self._default_store = None
+        pt = self._upload_parts(self, built)
+        self._parts = pt
         self._parts_cfg = dict(tets_per_part=tets_per_part, parts=parts)
         self.parts_per_mesh = [r["parts"] for r in built]
         return pt
@@ -1059,11 +1068,11 @@ class SimModelDO:
             return 1 << 30
         return per
 
-    def _cut_default(self) -> None:
-        """(Re)cut the default frame's partition."""
+    def _build_default(self) -> None:
+        """(Re)cut the default frame's partition and upload it."""
         if self._default_store is not None:
             torch.cuda.synchronize(self.device)  # frames in flight on any stream read the tables
-        self._default_store = self._default_built = None
+        self._default_store = None
         self._default_modes = self._modes()
         per_part = self._default_tets_per_part()
         if per_part is None:
@@ -1075,7 +1084,9 @@ class SimModelDO:
         nxcd = int(lib.ffsrl_xcd_count())
         cus = torch.cuda.get_device_properties(self.x.device).multi_processor_count
         if nxcd > 0 and max(r["parts"] for r in built) <= min(cus // nxcd, PART_MAX):
-            self._default_built = built
+            store = SimpleNamespace()
+            store.pt = self._upload_parts(store, built)
+            self._default_store = store
 
     def default_parts(self) -> Optional[Parts]:
         """The partition that ``SimIntegratorDO``'s default frame uses (None: one
@@ -1084,11 +1095,7 @@ class SimModelDO:
         if getattr(self, "_parts", None) is not None or not self.x.is_cuda or torch.cuda.is_current_stream_capturing():
             return None
         if self._default_modes != self._modes():
-            self._cut_default()
-        if self._default_built is not None:
-            store = SimpleNamespace()
-            store.pt = self._upload_parts(store, self._default_built)
-            self._default_store, self._default_built = store, None
+            self._build_default()
         return None if self._default_store is None else self._default_store.pt
 
     @property

@@ -113,7 +113,7 @@ class SceneServer:
         slot_class = np.repeat(np.arange(len(self.classes)), self.capacity)
         tips = np.asarray(tips, np.float32).reshape(len(self.classes), 4, 3)
         self.model = SimModelDO(self.classes, slot_class.tolist(), device=device, tips=tips[slot_class],
-                                **model_kwargs)
+                                **{"default_partition": False, **model_kwargs})
         m = self.model
         self.slot_class = slot_class
         self.n_slots = int(slot_class.size)

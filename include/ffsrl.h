@@ -285,7 +285,8 @@ typedef struct ffsrl_parts {
                                      pass; NULL without it) */
   uint64_t* sums;                 /* [3][stride][2] fixed-point sums of shared vertices, by state
                                      vertex; zero before the first frame, left zero by every frame */
-  int64_t stride;                 /* vertices per plane of sums (>= every env's vbase + nv) */
+  int64_t stride;                 /* vertices per plane of sums (>= vbase + nv of every env in
+                                     several parts) */
   uint32_t* ctr;                  /* [4 n_env + 64]: counters in the first 4 n_env + 17 words (zero
                                      before the first frame, left zero by every frame), then the
                                      claim table's extent per XCD (written by every launch) */
