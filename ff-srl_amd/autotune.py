@@ -104,7 +104,7 @@ class Autotuner:
         order = model.dispatch_order().data_ptr() if cfg["dispatch"] == "lpt" else None
         s = stream.cuda_stream
         if cfg.get("parts"):
-            if getattr(model, "_parts_cfg", {}).get("tets_per_part") != cfg["parts"]:
+            if model.parts_cfg.get("tets_per_part") != cfg["parts"]:
                 model.enable_parts(tets_per_part=cfg["parts"])
             run = lambda: lib.ffsrl_frame_parts(model.batch, model.params, model.parts, order, model.numEnvs, 1, s)
         elif cfg.get("shared"):
@@ -131,6 +131,7 @@ class Autotuner:
             self.apply(model, cfg)
             return cfg
         stream = torch.cuda.current_stream(model.device)
+        own = model.parts_cfg
         orig = (model.topo[0].constraint_order, model.topo[0].chunk) if model.topo else ("local", LOCAL_CHUNK)
         state = [(t, t.clone()) for t in self._state(model)]
         lam0 = [(t, t.clone()) for t in self._lambdas(model)]
@@ -156,6 +157,10 @@ class Autotuner:
             t.copy_(saved)
         results.sort(key=lambda r: r[0])
         best = dict(results[0][1])
+        if not best["parts"] and model.parts_cfg != own:  # the model's own partition, or none, as before the trials
+            model.disable_parts()
+            if own:
+                model.enable_parts(**own)
         self.apply(model, best)
         torch.cuda.synchronize(model.device)
         self.cache[key] = {"best": best, "ms": results[0][0],
@@ -168,5 +173,5 @@ class Autotuner:
         t = model.topo[0] if model.topo else None
         if t is not None and (t.constraint_order != "local" or t.chunk != cfg["chunk"]):
             model.set_constraint_order("local", cfg["chunk"])
-        if cfg.get("parts") and getattr(model, "_parts_cfg", {}).get("tets_per_part") != cfg["parts"]:
+        if cfg.get("parts") and model.parts_cfg.get("tets_per_part") != cfg["parts"]:
             model.enable_parts(tets_per_part=cfg["parts"])

@@ -1046,6 +1046,17 @@ class SimModelDO:
         self.parts_per_mesh = [r["parts"] for r in built]
         return pt
 
+    def disable_parts(self) -> None:
+        """Give up the partition of ``enable_parts``: the default frame uses the
+        model's own again (``default_parts``)."""
+        if getattr(self, "_parts", None) is None:
+            return
+        torch.cuda.synchronize(self.device)  # frames in flight on any stream read the tables
+        self._parts = self._parts_cfg = self.parts_per_mesh = None
+        self._parts_host = self.p_rows = self.p_env = self.p_verts = self.p_tets16 = self.p_edges16 = None
+        self.p_tris16 = self.p_sums = self.p_ctr = self.p_claims = None
+        self._default_modes = None           # freed by enable_parts
+
     def _default_tets_per_part(self) -> Optional[int]:
         """Tets per part of the default frame's own partition, or None where
         the default frame keeps one workgroup per env (``ffsrl_frame``), by
@@ -1097,6 +1108,11 @@ class SimModelDO:
         if self._default_modes != self._modes():
             self._build_default()
         return None if self._default_store is None else self._default_store.pt
+
+    @property
+    def parts_cfg(self) -> dict:
+        """The arguments of the last ``enable_parts`` (empty without a partition of the model's own)."""
+        return dict(getattr(self, "_parts_cfg", None) or {})
 
     @property
     def parts(self) -> Parts:

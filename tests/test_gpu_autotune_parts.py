@@ -1,0 +1,55 @@
+"""What tuning leaves behind: the model's partition as it was unless a
+partitioned frame is the choice."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+KW = dict(simSubsteps=8, distance="xpbd", volume="xpbd")
+
+
+def _model(pkg, gpu, tets, n):
+    return pkg.SimModelDO([pkg.scenes.solid("ellipsoid", tets, seed=17)], [0] * n, device=gpu, **KW)
+
+
+@pytest.mark.parametrize("own", [None, dict(tets_per_part=700, parts=None)])
+def test_partition_is_as_before_when_no_parts_win(pkg, gpu, own, monkeypatch):
+    A = pkg.autotune
+    a, b = (_model(pkg, gpu, 9000, 6) for _ in range(2))
+    if own:
+        b.enable_parts(**own)
+    had_default = b._default_store is not None
+    # timings of a device on which one workgroup per env wins
+    real = A.Autotuner._time
+    monkeypatch.setattr(A.Autotuner, "_time", staticmethod(
+        lambda model, cfg, frames, stream: real(model, cfg, frames, stream) + (1e3 if cfg["parts"] else 0.0)
+        + (1e3 if cfg["shared"] else 0.0)))
+    cfg = A.Autotuner().tune(b, frames=1)
+    assert not cfg["parts"] and not cfg["shared"]
+    assert b.parts_cfg == (own or {}) and (getattr(b, "_parts", None) is not None) == bool(own)
+    integ = pkg.SimIntegratorDO(gpu)
+    integ.stepModel(b, refit=True)              # an integrator that is not tuned
+    assert (b._default_store is not None) == had_default
+    pkg.lib.ffsrl_frame(a.batch, a.params, None, 1024, 1, a.stream())
+    if own:
+        pkg.SimIntegratorDO(gpu, parts=True).stepModel(b, refit=True)
+        pkg.lib.ffsrl_frame(a.batch, a.params, None, 1024, 1, a.stream())
+    torch.cuda.synchronize()
+    assert torch.equal(a.x, b.x) and torch.equal(a.v, b.v)
+
+
+def test_disable_parts(pkg, gpu):
+    a, b = (_model(pkg, gpu, 20000, 5) for _ in range(2))
+    assert b._default_store is not None
+    base = torch.cuda.memory_allocated(gpu)
+    integ = pkg.SimIntegratorDO(gpu)
+    for k in range(3):
+        b.enable_parts(tets_per_part=3000)
+        assert b.default_parts() is None
+        pkg.SimIntegratorDO(gpu, parts=True).stepModel(b)
+        b.disable_parts()
+        assert b.default_parts() is not None and b.parts_cfg == {}
+        integ.stepModel(b)
+        for _ in range(2):
+            pkg.lib.ffsrl_frame(a.batch, a.params, None, 1024, 0, a.stream())
+    torch.cuda.synchronize()
+    assert torch.equal(a.x, b.x) and torch.cuda.memory_allocated(gpu) <= base + (1 << 20)
