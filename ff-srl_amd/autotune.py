@@ -13,13 +13,14 @@ Knobs (all leave the results unchanged; the frame's Jacobi sums are integers):
             many envs as CUs;
   parts     the partitioned frame (each env's constraints cut into parts,
             one 1024-thread workgroup per part with the part's state in
-            LDS): 0 (not partitioned), or the tets per part (PART_WHOLE:
-            as few parts as a workgroup's LDS allows).
+            LDS): 0 (not partitioned), the tets per part (PART_WHOLE: as
+            few parts as a workgroup's LDS allows), or PART_DEFAULT (the
+            default frame's own partition, where it uses one).
 
 A trial runs whole frames on a snapshot of the state, which is restored
 afterwards, so tuning does not advance the simulation.  The cache is a JSON
 file; its key is (env-count bucket, mean-tets bucket, max-tets bucket,
-constraint set), buckets being powers of two.
+constraint set, KERNELS), buckets being powers of two.
 """
 from __future__ import annotations
 
@@ -40,15 +41,19 @@ DISPATCH = ("lpt", "table")
 CHUNKS = (64, 128, 256)
 PART_WHOLE = 1 << 30
 PART_SIZES = (PART_WHOLE, PART_TETS)
+PART_DEFAULT = "default"
+KERNELS = 3  # the kernels that the cached times are of: counted up when a frame form or its speed changes
 DEFAULT = {"block": 1024, "dispatch": "lpt", "chunk": LOCAL_CHUNK, "shared": False, "parts": 0}
 
 
 def parts_candidates(model: SimModelDO) -> tuple:
     """(0,) or (0, *PART_SIZES): the partitioned frame (tets per part; 0 =
-    not partitioned) is a candidate where the device has an XCD map."""
+    not partitioned) is a candidate where the device has an XCD map.  So is the
+    frame that an integrator without a tuned shape would run, where it is
+    partitioned: the choice is then no slower than no choice."""
     if lib.ffsrl_xcd_count() <= 0:
         return (0,)
-    return (0,) + PART_SIZES
+    return (0,) + PART_SIZES + ((PART_DEFAULT,) if model.default_parts() is not None else ())
 
 
 def shared_candidates(model: SimModelDO) -> tuple:
@@ -70,7 +75,7 @@ def key_of(model: SimModelDO) -> str:
     run on this device (an XCD map)."""
     tets = np.array([model.meshes[k].num_tets for k in model.env_mesh], dtype=np.float64)
     flags = (f"d{model.dist_mode}v{model.vol_mode}n{int(model.nh_on)}s{model.simSubsteps}i{model.simConstraints}"
-             f"c{int(model.collision)}x{int(lib.ffsrl_xcd_count() > 0)}k2")
+             f"c{int(model.collision)}x{int(lib.ffsrl_xcd_count() > 0)}k{KERNELS}")
     return f"envs{_bucket(model.numEnvs)}-tets{_bucket(tets.mean())}-max{_bucket(tets.max())}-{flags}"
 
 
@@ -103,7 +108,13 @@ class Autotuner:
     def _time(model: SimModelDO, cfg: dict, frames: int, stream) -> float:
         order = model.dispatch_order().data_ptr() if cfg["dispatch"] == "lpt" else None
         s = stream.cuda_stream
-        if cfg.get("parts"):
+        if cfg.get("parts") == PART_DEFAULT:
+            model.disable_parts()                 # the trials before
+            plan = model.default_parts()
+            if plan is None:
+                raise ValueError("the default frame is not partitioned")
+            run = lambda: lib.ffsrl_frame_parts(model.batch, model.params, plan, order, model.numEnvs, 1, s)
+        elif cfg.get("parts"):
             if model.parts_cfg.get("tets_per_part") != cfg["parts"]:
                 model.enable_parts(tets_per_part=cfg["parts"])
             run = lambda: lib.ffsrl_frame_parts(model.batch, model.params, model.parts, order, model.numEnvs, 1, s)
@@ -133,6 +144,7 @@ class Autotuner:
         stream = torch.cuda.current_stream(model.device)
         own = model.parts_cfg
         orig = (model.topo[0].constraint_order, model.topo[0].chunk) if model.topo else ("local", LOCAL_CHUNK)
+        candidates = parts_candidates(model)
         state = [(t, t.clone()) for t in self._state(model)]
         lam0 = [(t, t.clone()) for t in self._lambdas(model)]
         results = []
@@ -141,8 +153,10 @@ class Autotuner:
             lam = [(t, t.clone()) for t in self._lambdas(model)]
             torch.cuda.synchronize(model.device)
             for block, dispatch, shared, parts in itertools.product(BLOCKS, DISPATCH, shared_candidates(model),
-                                                                    parts_candidates(model)):
+                                                                    candidates):
                 if parts and (block != 1024 or shared):   # the partitioned frame runs 1024-thread parts
+                    continue
+                if parts == PART_DEFAULT and dispatch != DEFAULT["dispatch"]:
                     continue
                 cfg = {"block": block, "dispatch": dispatch, "chunk": chunk, "shared": shared, "parts": parts}
                 try:
@@ -157,7 +171,7 @@ class Autotuner:
             t.copy_(saved)
         results.sort(key=lambda r: r[0])
         best = dict(results[0][1])
-        if not best["parts"] and model.parts_cfg != own:  # the model's own partition, or none, as before the trials
+        if best["parts"] in (0, PART_DEFAULT) and model.parts_cfg != own:  # the model's own partition, or none, as before the trials
             model.disable_parts()
             if own:
                 model.enable_parts(**own)
@@ -173,5 +187,5 @@ class Autotuner:
         t = model.topo[0] if model.topo else None
         if t is not None and (t.constraint_order != "local" or t.chunk != cfg["chunk"]):
             model.set_constraint_order("local", cfg["chunk"])
-        if cfg.get("parts") and model.parts_cfg.get("tets_per_part") != cfg["parts"]:
+        if cfg.get("parts") not in (None, 0, PART_DEFAULT) and model.parts_cfg.get("tets_per_part") != cfg["parts"]:
             model.enable_parts(tets_per_part=cfg["parts"])

@@ -49,8 +49,9 @@ class SimIntegratorDO:
         self.block = int(cfg["block"])
         self.dispatch_sorted = cfg["dispatch"] == "lpt"
         self.shared = bool(cfg.get("shared", False))
-        self.parts = bool(cfg.get("parts", False))
-        self.tuned = True
+        default = cfg.get("parts") == "default"   # the model's own partition, as without tuning
+        self.parts = bool(cfg.get("parts", False)) and not default
+        self.tuned = not default
 
     def autotune(self, simModel: SimModelDO, cache_path=None, frames: int = 2) -> dict:
         """Tune (or look up) the launch shape for this batch and use it."""

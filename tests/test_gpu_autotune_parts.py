@@ -53,3 +53,35 @@ def test_disable_parts(pkg, gpu):
             pkg.lib.ffsrl_frame(a.batch, a.params, None, 1024, 0, a.stream())
     torch.cuda.synchronize()
     assert torch.equal(a.x, b.x) and torch.cuda.memory_allocated(gpu) <= base + (1 << 20)
+
+
+def test_choice_is_no_slower_than_no_choice(pkg, gpu, tmp_path, monkeypatch):
+    """The default frame's own partition is timed, may be chosen and is then what
+    the tuned integrator runs; a cache written for other kernels is not used."""
+    A = pkg.autotune
+    a, b = (_model(pkg, gpu, 20000, 5) for _ in range(2))
+    cache = str(tmp_path / "tune.json")
+    old = A.Autotuner(cache)
+    old.cache[A.key_of(b).replace(f"k{A.KERNELS}", f"k{A.KERNELS - 1}")] = {
+        "best": {"block": 256, "dispatch": "table", "chunk": 64, "shared": False, "parts": 0}}
+    old.save()
+    real = A.Autotuner._time
+    monkeypatch.setattr(A.Autotuner, "_time", staticmethod(
+        lambda model, cfg, frames, stream: real(model, cfg, frames, stream) + (1e3 if cfg["parts"] != "default" else 0.0)))
+    integ = pkg.SimIntegratorDO(gpu)
+    cfg = integ.autotune(b, cache_path=cache, frames=1)
+    assert cfg["parts"] == "default" and cfg["block"] == 1024 and cfg["dispatch"] == "lpt" and not cfg["shared"]
+    assert b.parts_cfg == {} and not integ.parts and not integ.tuned
+    calls = []
+    run = pkg.lib.ffsrl_frame_parts
+    monkeypatch.setattr(type(pkg.lib), "ffsrl_frame_parts", lambda self, *x: calls.append(x[2]) or run(*x), raising=False)
+    integ.stepModel(b, refit=True)
+    monkeypatch.undo()
+    assert len(calls) == 1
+    again = pkg.SimIntegratorDO(gpu)
+    assert again.autotune(b, cache_path=cache) == cfg
+    again.stepModel(b, refit=True)
+    for _ in range(2):
+        pkg.lib.ffsrl_frame(a.batch, a.params, None, 1024, 1, a.stream())
+    torch.cuda.synchronize()
+    assert torch.equal(a.x, b.x) and torch.equal(a.bvh_lo, b.bvh_lo)
