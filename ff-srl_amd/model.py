@@ -1069,11 +1069,14 @@ class SimModelDO:
         cus = torch.cuda.get_device_properties(self.x.device).multi_processor_count
         per = default_tets_per_part(items, [m.num_vertices for m in self.meshes], self.env_mesh, cus,
                                     int(lib.ffsrl_xcd_count()), collide, p.substeps * p.iterations)
-        # A full chip, each env in one part: its positions in LDS instead of global memory.  Faster with
-        # Neo-Hookean, whose inverse rest matrices fill the caches (us, one workgroup per env / one part:
-        # 20k tets x 1024 envs, one iteration 3146 / 2931, two 7081 / 6204; 1.5k x 256 105 / 103), except with
-        # collision and two iterations (7831 / 8240, registers); slower without (volume and distance 2356 / 2572)
-        # and on an idle chip (4k x 4 168 / 171: the claim table's launch).
+        # A full chip, each env in one part: its positions in LDS instead of global memory.  Always faster with
+        # Neo-Hookean, whose inverse rest matrices fill the caches (10 substeps, us, one workgroup per env / one
+        # part: 20k tets x 1024 envs, one iteration 3006 / 2833, two 6714 / 5882; 1.5k x 256 106 / 93); with
+        # collision and two iterations too (7547 / 7050), where it is not used yet: the claimed form was slower
+        # (8240).  Without Neo-Hookean it depends: volume and distance, one iteration, 1.5k x 1024 287 / 277, 5k
+        # 672 / 704, 20k 2354 / 2547, the liver scene's frame and render 712 / 647; with collision 5k 840 / 820, 20k
+        # 2728 / 2739; carried multipliers, two iterations, 1.5k 559 / 491, 5k 1429 / 1344, 20k 5202 / 5019: one
+        # workgroup per env is kept for all of these.
         if (per is None and p.nh_on and self.numEnvs >= cus and not (collide and p.iterations > 1)
                 and self.max_nv <= int(lib.ffsrl_parts_max_solo())):
             return 1 << 30
