@@ -17,7 +17,8 @@ Knobs (all leave the results unchanged; the frame's Jacobi sums are integers):
             few parts as a workgroup's LDS allows), or PART_DEFAULT (the
             default frame's own partition, where it uses one).
 
-A trial runs whole frames on a snapshot of the state, which is restored
+A trial runs whole frames (at least ``frames``, for about TRIAL_MS after as
+many unmeasured ones) on a snapshot of the state, which is restored
 afterwards, so tuning does not advance the simulation.  The cache is a JSON
 file; its key is (env-count bucket, mean-tets bucket, max-tets bucket,
 constraint set, KERNELS), buckets being powers of two.
@@ -42,6 +43,9 @@ CHUNKS = (64, 128, 256)
 PART_WHOLE = 1 << 30
 PART_SIZES = (PART_WHOLE, PART_TETS)
 PART_DEFAULT = "default"
+# A trial's frames, and those before it, take about this long.  Of a device that was idle the first frames are
+# slower by more than the candidates differ: 1024 mixed envs 2.33 ... 2.38 ms for forms of 1.91 ... 2.16.
+TRIAL_MS = 15.0
 KERNELS = 3  # the kernels that the cached times are of: counted up when a frame form or its speed changes
 DEFAULT = {"block": 1024, "dispatch": "lpt", "chunk": LOCAL_CHUNK, "shared": False, "parts": 0}
 
@@ -123,14 +127,19 @@ class Autotuner:
             run = lambda: lib.ffsrl_frame_shared(model.batch, model.params, order, model.numEnvs, cfg["block"], 1, s)
         else:
             run = lambda: lib.ffsrl_frame(model.batch, model.params, order, cfg["block"], 1, s)
+        def ms(n: int) -> float:
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record(stream)
+            for _ in range(n):
+                run()
+            e1.record(stream)
+            e1.synchronize()
+            return e0.elapsed_time(e1) / n
+
         run()                                                                           # warm
-        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        e0.record(stream)
-        for _ in range(frames):
-            run()
-        e1.record(stream)
-        e1.synchronize()
-        return e0.elapsed_time(e1) / frames
+        n = max(frames, min(200, math.ceil(TRIAL_MS / max(ms(1), 1e-3))))
+        ms(n)                                     # the clocks of the idle device rise
+        return ms(n)
 
     def tune(self, model: SimModelDO, frames: int = 2, force: bool = False) -> dict:
         """Best {block, dispatch, chunk, shared, parts} for this batch (cached),

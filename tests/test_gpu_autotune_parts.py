@@ -85,3 +85,13 @@ def test_choice_is_no_slower_than_no_choice(pkg, gpu, tmp_path, monkeypatch):
         pkg.lib.ffsrl_frame(a.batch, a.params, None, 1024, 1, a.stream())
     torch.cuda.synchronize()
     assert torch.equal(a.x, b.x) and torch.equal(a.bvh_lo, b.bvh_lo)
+
+
+def test_trials_are_long_enough(pkg, gpu, monkeypatch):
+    """A trial of short frames runs many of them, measured after as many that are not."""
+    A = pkg.autotune
+    m = _model(pkg, gpu, 900, 2)
+    run, calls = pkg.lib.ffsrl_frame, []
+    monkeypatch.setattr(type(pkg.lib), "ffsrl_frame", lambda self, *x: calls.append(1) or run(*x), raising=False)
+    ms = A.Autotuner._time(m, dict(A.DEFAULT), 2, torch.cuda.current_stream(gpu))
+    assert 0 < ms < 1.0 and (len(calls) - 2) / 2 >= min(200, A.TRIAL_MS / 1.0)
