@@ -1567,13 +1567,13 @@ __device__ __forceinline__ void solo_env(const ffsrl_batch& b, const ffsrl_param
   if (refit) refit_env<BLOCK>(b, e);
 }
 
-// Polls (of about a microsecond) without a workgroup of this launch at work on
+// Polls (of about two microseconds) without a workgroup of this launch at work on
 // the XCD after which the parts of an env that k_frame_rest can run withdraw.
 // In a launch that has the device to itself an env's missing parts are claimed
 // as soon as workgroups finish what they work on, so only a launch held back by
 // others gets there.  The parts of a larger env wait as long as share_wait does:
 // another stream's kernel may hold the CUs for longer than that.
-constexpr int kAssemblePolls = 1 << 11;
+constexpr int kAssemblePolls = 1 << 10;
 
 // The assembly word (parts_wait.hpp) of an env.  Claims are in slot order, so
 // every part of the envs of the XCD's earlier claims has been claimed, and of
@@ -1588,11 +1588,11 @@ struct AssemblyWord {
   uint32_t* word;
   __device__ uint32_t add(uint32_t n) { return atomicAdd(word, n); }
   __device__ uint32_t cas(uint32_t expected, uint32_t desired) { return atomicCAS(word, expected, desired); }
-  __device__ bool idle() {  // one claim further with each call
-    const int env = *claims >> 6;
+  __device__ bool idle() {  // one env further with each call
+    const int env = *claims >> 6, np = env_parts[2 * env + 1];
     uint32_t* c = ctr + 4 * (int64_t)env;
     if (&c[3] == word) return true;
-    if (atomicAdd(&c[0], 0u) >= (uint32_t)env_parts[2 * env + 1] || (atomicAdd(&c[3], 0u) & kWithdrawn)) ++claims;
+    if (atomicAdd(&c[0], 0u) >= (uint32_t)np || (atomicAdd(&c[3], 0u) & kWithdrawn)) claims += np;
     return false;
   }
   // After the first polls the wait is for workgroups to come free: fewer polls
