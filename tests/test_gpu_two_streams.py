@@ -64,3 +64,36 @@ def test_every_env_in_one_part(pkg, gpu, mode, listed):
         assert (s is None and t is None) or torch.equal(s, t), k
     if mode == "collision":
         assert int(a.laparoscopeInCollision.sum()) > 0
+
+
+@pytest.mark.parametrize("large", [False, True])
+def test_frame_beside_a_launch_that_holds_the_cus(pkg, gpu, large):
+    """Another stream's frame holds all but a few CUs for about 20 ms: parts that
+    cannot come together beside it withdraw and their envs are run by one
+    workgroup each; an env that only its parts can run waits for the CUs."""
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    hold = pkg.SimModelDO([pkg.scenes.solid("ellipsoid", 20000, seed=5)], [0] * (cus - 8), device=gpu, simSubsteps=400,
+                          distance="pbd", volume="pbd")
+    kw = dict(simSubsteps=6, distance="pbd", volume="pbd")
+    mesh = pkg.scenes.cube_grid(23) if large else pkg.scenes.solid("ellipsoid", 20000, seed=6)
+    n = 2 if large else 16
+    ref, got = (pkg.SimModelDO([mesh], [0] * n, device=gpu, default_partition=False, **kw) for _ in range(2))
+    for m in (ref, got):
+        m.enable_parts(tets_per_part=1 << 30 if large else 1280)
+        assert int(m._parts_host[:, 1].max()) > 2 and (m.max_nv > pkg.lib.ffsrl_frame_max_vertices()) == large
+    integ = pkg.SimIntegratorDO(gpu, parts=True)
+    orders = [m.dispatch_order() for m in (hold, ref, got)]
+    a, b = torch.cuda.Stream(gpu), torch.cuda.Stream(gpu)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        pkg.lib.ffsrl_frame(hold.batch, hold.params, orders[0].data_ptr(), 1024, 0, hold.stream())
+    with torch.cuda.stream(b):
+        for _ in range(2):
+            integ.stepModel(got, refit=True)
+    torch.cuda.synchronize()
+    for _ in range(2):                      # the device to itself
+        integ.stepModel(ref, refit=True)
+    torch.cuda.synchronize()
+    assert int(got.frame_status().abs().sum()) == 0 and int(got.p_ctr[:4 * n + 32].abs().sum()) == 0
+    assert int(got.p_sums.abs().sum()) == 0
+    assert all(torch.equal(getattr(ref, k), getattr(got, k)) for k in ("x", "v", "p", "bvh_lo", "bvh_hi"))
